@@ -67,8 +67,8 @@ extern "C" {
  * hipMemcpyAsync for copy, scale_kernel<T> / triad_kernel<T> otherwise.
  *
  * dst, b: n elements of `dtype`; c: n elements for TRIAD, ignored (may be NULL)
- * otherwise. Any n (0 is a no-op) and any element alignment: 16-byte aligned
- * buffers take the vector kernel plus a scalar tail, others a scalar kernel.
+ * otherwise. Any n (0 is a no-op) and any alignment: 16-byte chunks from dst's
+ * first 16-byte boundary on, the elements before and after them one by one.
  * Arithmetic: fp32 math with one round-to-nearest-even to the element type
  * (fp64 math for float64); TRIAD is one fused multiply-add, fma(s, c, b).
  * blocks_per_cu: grid = min(CUs * blocks_per_cu, work); <= 0 selects the

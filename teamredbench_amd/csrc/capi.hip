@@ -461,7 +461,7 @@ int mb_kernel_info(int kind, int a, int b, int64_t m, int64_t n, int64_t k, char
         if ((rc = stream_plan(op, dtype, dummy, dummy, dummy, (uint64_t)m, (int)n, *props, &plan)) !=
             MB_OK)
             return rc;
-        j.str("implementation", plan.vector_path ? "gfx950_stream_dwordx4" : "gfx950_stream_scalar");
+        j.str("implementation", "gfx950_stream_dwordx4");
         j.num("threads_per_block", plan.threads);
         j.num("vector_unroll", plan.chunks_per_trip);
         j.num("blocks_per_cu", plan.blocks_per_cu);

@@ -92,12 +92,12 @@ inline const char* dtype_name(int dtype) {
 // ---- internal launch interfaces (one per translation unit) -----------------
 
 struct StreamPlan {
-    bool vector_path = false;   // 16-byte chunk kernel (else scalar kernel)
     int threads = 0;
     int blocks = 0;
     int blocks_per_cu = 0;
     int chunks_per_trip = 0;    // 16-byte chunks per thread per loop trip
     bool nontemporal = false;
+    uint64_t head = 0;          // elements before the vector body
     uint64_t chunks = 0;        // 16-byte chunks in the vector body
     uint64_t tail = 0;          // elements after the vector body
     uint64_t span = 0;          // chunks per block (0 = grid-stride schedule)

@@ -134,7 +134,7 @@ struct ChunkOp<MB_OP_TRIAD, MB_DT_FLOAT64> {
     }
 };
 
-// ---- scalar element arithmetic (tails and unaligned buffers) ----------------
+// ---- scalar element arithmetic (heads and tails) -----------------------------
 
 template <int DT>
 struct Scalar;
@@ -202,14 +202,17 @@ __device__ inline void scalar_element(void* dst, const void* b, const void* c, u
 
 // ---- kernels ---------------------------------------------------------------
 
+// Sixteen bytes at any address.
+typedef u32x4 u32x4_any __attribute__((aligned(1)));
+
 template <bool NT>
-__device__ inline u32x4 load_chunk(const u32x4* p) {
+__device__ inline u32x4 load_chunk(const u32x4_any* p) {
     if (NT) return __builtin_nontemporal_load(p);
     return *p;
 }
 
 template <bool NT>
-__device__ inline void store_chunk(u32x4* p, u32x4 v) {
+__device__ inline void store_chunk(u32x4_any* p, u32x4 v) {
     if (NT) {
         __builtin_nontemporal_store(v, p);
     } else {
@@ -217,18 +220,28 @@ __device__ inline void store_chunk(u32x4* p, u32x4 v) {
     }
 }
 
-// Vector body over `chunks` 16-byte chunks, then the `tail` trailing elements
-// (fewer than one chunk) handled by the first threads of the grid.
+// Vector body over `chunks` 16-byte chunks that start `head` elements into
+// the arrays, then the `edge` elements outside it (a head of less than a
+// 128-byte line, a tail of less than a chunk) by the grid's first threads.
 // span == 0: grid-stride -- consecutive trips of a thread are one grid apart.
 // span  > 0: each block walks its own contiguous run of `span` chunks, the
 //            block's lanes side by side, trips one block-width apart.
+// Chunks need no alignment: gfx950 loads and stores 16 bytes at any address
+// (u32x4_any), with the instructions it uses for aligned ones. The plan picks
+// `head` so that dst's chunks are aligned; b and c then start wherever they
+// do. Bound: HBM, as with aligned arrays. On MI355X, source one element off,
+// against one element per lane and load (the kernel such arrays had before):
+// fp16 copy of 5e7 elements 294 -> 36 us (aligned 36), bf16 scale of 6e7 374
+// -> 43 (42), fp32 triad of 2e8 1490 -> 388 (381), int8 copy of 4e8 2240 ->
+// 134 (128).
 template <int OP, int DT, int U, bool NT>
 __global__ void __launch_bounds__(1024)
 stream_vec_kernel(void* __restrict__ dst, const void* __restrict__ b, const void* __restrict__ c,
-                  uint64_t chunks, uint64_t tail, uint64_t span, float s, double sd) {
-    const u32x4* B = static_cast<const u32x4*>(b);
-    const u32x4* C = static_cast<const u32x4*>(c);
-    u32x4* D = static_cast<u32x4*>(dst);
+                  uint64_t chunks, unsigned head, unsigned edge, uint64_t span, float s, double sd) {
+    constexpr int esize = (DT == MB_DT_FLOAT32) ? 4 : (DT == MB_DT_FLOAT64) ? 8 : (DT == MB_DT_INT8) ? 1 : 2;
+    const u32x4_any* B = reinterpret_cast<const u32x4_any*>(static_cast<const char*>(b) + head * esize);
+    const u32x4_any* C = reinterpret_cast<const u32x4_any*>(static_cast<const char*>(c) + head * esize);
+    u32x4_any* D = reinterpret_cast<u32x4_any*>(static_cast<char*>(dst) + head * esize);
     const uint64_t tid = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
     uint64_t stride, end, i;
     if (span == 0) {
@@ -262,27 +275,12 @@ stream_vec_kernel(void* __restrict__ dst, const void* __restrict__ b, const void
         if (OP == MB_OP_TRIAD) vc = load_chunk<NT>(C + i);
         store_chunk<NT>(D + i, ChunkOp<OP, DT>::apply(vb, vc, s, sd));
     }
-    if (tid < tail) {
-        const int esize = (DT == MB_DT_FLOAT32) ? 4 : (DT == MB_DT_FLOAT64) ? 8 : (DT == MB_DT_INT8) ? 1 : 2;
-        const uint64_t first = chunks * (16 / esize);
-        scalar_element<OP, DT>(dst, b, c, first + tid, s, sd);
-    }
-}
-
-// Element-wise grid-stride kernel for buffers that are not 16-byte aligned.
-template <int OP, int DT>
-__global__ void __launch_bounds__(1024)
-stream_scalar_kernel(void* __restrict__ dst, const void* __restrict__ b, const void* __restrict__ c,
-                     uint64_t n, float s, double sd) {
-    const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
-    for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride)
-        scalar_element<OP, DT>(dst, b, c, i, s, sd);
+    if (tid < edge) scalar_element<OP, DT>(dst, b, c, tid < head ? tid : chunks * (16 / esize) + tid, s, sd);
 }
 
 // ---- dispatch --------------------------------------------------------------
 
-typedef void (*VecKernel)(void*, const void*, const void*, uint64_t, uint64_t, uint64_t, float, double);
-typedef void (*ScalarKernel)(void*, const void*, const void*, uint64_t, float, double);
+typedef void (*VecKernel)(void*, const void*, const void*, uint64_t, unsigned, unsigned, uint64_t, float, double);
 
 template <int OP, int DT>
 VecKernel pick_vec(int u, bool nt) {
@@ -323,25 +321,6 @@ VecKernel vec_kernel_for(int op, int dtype, int u, bool nt) {
             case MB_DT_FLOAT64: return pick_vec<MB_OP_TRIAD, MB_DT_FLOAT64>(u, nt);
         }
     }
-    return nullptr;
-}
-
-template <int OP>
-ScalarKernel scalar_for_dtype(int dtype) {
-    switch (dtype) {
-        case MB_DT_FLOAT32: return stream_scalar_kernel<OP, MB_DT_FLOAT32>;
-        case MB_DT_BFLOAT16: return stream_scalar_kernel<OP, MB_DT_BFLOAT16>;
-        case MB_DT_FLOAT16: return stream_scalar_kernel<OP, MB_DT_FLOAT16>;
-        case MB_DT_FLOAT64: return stream_scalar_kernel<OP, MB_DT_FLOAT64>;
-        case MB_DT_INT8: return OP == MB_OP_COPY ? stream_scalar_kernel<OP, MB_DT_INT8> : nullptr;
-    }
-    return nullptr;
-}
-
-ScalarKernel scalar_kernel_for(int op, int dtype) {
-    if (op == MB_OP_COPY) return scalar_for_dtype<MB_OP_COPY>(dtype);
-    if (op == MB_OP_SCALE) return scalar_for_dtype<MB_OP_SCALE>(dtype);
-    if (op == MB_OP_TRIAD) return scalar_for_dtype<MB_OP_TRIAD>(dtype);
     return nullptr;
 }
 
@@ -388,8 +367,6 @@ int knob_or(int knob, int fallback) {
     return v < 0 ? fallback : (int)v;
 }
 
-bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
-
 }  // namespace
 
 int stream_plan(int op, int dtype, const void* dst, const void* b, const void* c, uint64_t n,
@@ -418,34 +395,36 @@ int stream_plan(int op, int dtype, const void* dst, const void* b, const void* c
     plan->blocks_per_cu = bpc;
     plan->chunks_per_trip = u;
     plan->nontemporal = nt;
-    const bool vec = aligned16(dst) && aligned16(b) && (op != MB_OP_TRIAD || aligned16(c));
-    plan->vector_path = vec;
+    // Elements before dst's first 128-byte line, when whole elements reach it
+    // (the chunks of a dst off its own element size stay unaligned): every
+    // wave then stores whole lines. Chunks on a 16-byte boundary only left a
+    // partial line at both ends of every wave's store: dst one element off ran
+    // 235 us there and 198 here (fp32 copy of 1.5e8; aligned 193), 418 and
+    // 384 (fp32 triad of 2e8), 150 and 128 (int8 copy of 4e8).
+    constexpr uint64_t kLine = 128;
     const uint64_t per_chunk = 16 / (uint64_t)esize;
-    uint64_t work_items;
-    if (vec) {
-        plan->chunks = n / per_chunk;
-        plan->tail = n - plan->chunks * per_chunk;
-        work_items = (plan->chunks + (uint64_t)u - 1) / (uint64_t)u;
-        if (work_items < plan->tail) work_items = plan->tail;
-    } else {
-        plan->chunks = 0;
-        plan->tail = n;
-        work_items = n;
-    }
+    const uint64_t to_boundary = (kLine - reinterpret_cast<uintptr_t>(dst) % kLine) % kLine;
+    const uint64_t head = to_boundary % (uint64_t)esize == 0 ? to_boundary / (uint64_t)esize : 0;
+    plan->head = head < n ? head : n;
+    plan->chunks = (n - plan->head) / per_chunk;
+    plan->tail = n - plan->head - plan->chunks * per_chunk;
+    uint64_t work_items = (plan->chunks + (uint64_t)u - 1) / (uint64_t)u;
+    const uint64_t edge = plan->head + plan->tail;
+    if (work_items < edge) work_items = edge;
     uint64_t max_blocks = (uint64_t)props.cu_count * (uint64_t)bpc;
     uint64_t by_work = (work_items + (uint64_t)threads - 1) / (uint64_t)threads;
     uint64_t blocks = by_work < max_blocks ? by_work : max_blocks;
     if (blocks < 1) blocks = 1;
     plan->blocks = (int)blocks;
     plan->span = 0;
-    if (vec && sched == 1 && plan->chunks > 0) {
+    if (sched == 1 && plan->chunks > 0) {
         // Contiguous runs, a whole number of block-wide trips each.
         const uint64_t trip = (uint64_t)threads * (uint64_t)u;
         uint64_t span = (plan->chunks + blocks - 1) / blocks;
         span = (span + trip - 1) / trip * trip;
         plan->span = span;
         plan->blocks = (int)((plan->chunks + span - 1) / span);
-        if ((uint64_t)plan->blocks * threads < plan->tail) plan->blocks = (int)((plan->tail + threads - 1) / threads);
+        if ((uint64_t)plan->blocks * threads < edge) plan->blocks = (int)((edge + threads - 1) / threads);
     }
     return MB_OK;
 }
@@ -454,22 +433,13 @@ int stream_launch(int op, int dtype, void* dst, const void* b, const void* c, ui
                   double s, const StreamPlan& plan, hipStream_t stream) {
     if (n == 0) return MB_OK;
     const float sf = (float)s;
-    if (plan.vector_path) {
-        VecKernel k = vec_kernel_for(op, dtype, plan.chunks_per_trip, plan.nontemporal);
-        if (k == nullptr) {
-            set_error("no vector stream kernel for op %d dtype %d", op, dtype);
-            return MB_ERR_UNSUPPORTED;
-        }
-        hipLaunchKernelGGL(k, dim3(plan.blocks), dim3(plan.threads), 0, stream, dst, b, c,
-                           plan.chunks, plan.tail, plan.span, sf, s);
-    } else {
-        ScalarKernel k = scalar_kernel_for(op, dtype);
-        if (k == nullptr) {
-            set_error("no scalar stream kernel for op %d dtype %d", op, dtype);
-            return MB_ERR_UNSUPPORTED;
-        }
-        hipLaunchKernelGGL(k, dim3(plan.blocks), dim3(plan.threads), 0, stream, dst, b, c, n, sf, s);
+    VecKernel k = vec_kernel_for(op, dtype, plan.chunks_per_trip, plan.nontemporal);
+    if (k == nullptr) {
+        set_error("no stream kernel for op %d dtype %d", op, dtype);
+        return MB_ERR_UNSUPPORTED;
     }
+    hipLaunchKernelGGL(k, dim3(plan.blocks), dim3(plan.threads), 0, stream, dst, b, c, plan.chunks,
+                       (unsigned)plan.head, (unsigned)(plan.head + plan.tail), plan.span, sf, s);
     MB_HIP_TRY(hipGetLastError());
     return MB_OK;
 }

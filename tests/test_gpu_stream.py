@@ -85,6 +85,38 @@ def test_unaligned_buffers_take_the_scalar_kernel(lib, mode, dtype, offset):
     assert np.array_equal(_bits(got)[:offset], untouched)
 
 
+# (dst, source) byte offsets past a 128-byte line: heads of every length class, sources that share dst's
+# offset or not, and a dst off its own element size (no head reaches a line: its chunks stay unaligned).
+BYTE_OFFSETS = [(0, 1), (0, 8), (16, 0), (8, 8), (120, 24), (2, 127), (1, 0)]
+
+
+@pytest.mark.parametrize("mode, dtype", [("copy", "int8"), ("copy", "bfloat16"), ("scale", "float16"),
+                                         ("triad", "float32"), ("triad", "float64")])
+@pytest.mark.parametrize("dst_off, src_off", BYTE_OFFSETS)
+def test_arrays_at_any_address(lib, mode, dtype, dst_off, src_off):
+    # Lengths around the head (less than a line), one chunk after it, and several trips of the grid with a
+    # tail; bytes before and after dst stay as they were.
+    esize = torch.empty(0, dtype=rp.TORCH_DTYPES[dtype]).element_size()
+    stream = torch.cuda.current_stream().cuda_stream
+    for n in (1, 15, 128 // esize - 1, 128 // esize + 16 // esize + 1, 300_007):
+        print(f"[stream] any address {mode} {dtype} n={n} dst+{dst_off} src+{src_off}", flush=True)
+        b, c = rp.stream_inputs(n, dtype, seed=n)
+
+        def shifted(x):
+            raw = torch.zeros(n * esize + 256, dtype=torch.uint8)
+            raw[src_off:src_off + n * esize] = x.view(torch.uint8)
+            return raw.cuda()
+        db, dc = shifted(b), shifted(c)
+        dst = torch.full((n * esize + 512,), 0x5A, dtype=torch.uint8, device="cuda")
+        assert dst.data_ptr() % 128 == 0 and db.data_ptr() % 128 == 0
+        lib.stream(capi.OPS[mode], capi.DTYPES[dtype], dst.data_ptr() + dst_off, db.data_ptr() + src_off,
+                   dc.data_ptr() + src_off if mode == "triad" else None, n, 3.0, 0, stream)
+        got = dst.cpu().numpy()
+        exp = b.view(torch.uint8).numpy() if mode == "copy" else _expect(mode, dtype, b, c, 3.0).view(np.uint8)
+        assert np.array_equal(got[dst_off:dst_off + n * esize], exp)
+        assert (got[:dst_off] == 0x5A).all() and (got[dst_off + n * esize:] == 0x5A).all()
+
+
 def test_int8_copy(lib):
     b, c = rp.stream_inputs(100_003, "int8", seed=2)
     got = _run(lib, "copy", "int8", b, c, 1.0)
