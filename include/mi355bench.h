@@ -114,7 +114,8 @@ int mb_time_stream(int op, int dtype, void* dst, const void* b, const void* c,
  * (dtypes.py:24) but does not run natively (mfu_gemm.hip.cpp:9-21).
  * workspace: device scratch of at least mb_gemm_workspace_size() bytes (may
  * be NULL when that size is 0). The kernels leave it in a state the next
- * call can use without clearing.
+ * call can use without clearing. FLOAT32 / FLOAT64 use it to run faster (K
+ * split over idle CUs): with less than that size, or NULL, they run without.
  */
 int mb_gemm(int dtype, const void* A, const void* B, void* C, int64_t M,
             int64_t N, int64_t K, float scale_a, float scale_b, void* workspace,
@@ -128,8 +129,9 @@ size_t mb_gemm_workspace_size(int dtype, int64_t M, int64_t N, int64_t K);
  * cannot allocate device memory (code under HIP graph capture, serving loops,
  * harnesses that forbid hipMalloc). It has no counterpart in the reference.
  *
- * Same arguments, kernels and results as mb_gemm. The split-K / small-M
- * partial sums go to a library-owned device array of
+ * Same arguments, kernels and results as mb_gemm (as mb_gemm without a
+ * workspace for FLOAT32 / FLOAT64, which use no scratch here). The split-K /
+ * small-M partial sums go to a library-owned device array of
  * MB_NOALLOC_SCRATCH_BYTES per GPU, which each GPU holds until the process
  * ends; the call itself allocates nothing. Shapes whose plan needs more
  * scratch than that return MB_ERR_WORKSPACE before any launch. The first

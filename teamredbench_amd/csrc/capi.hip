@@ -130,6 +130,10 @@ int check_gemm_args(int dtype, const void* A, const void* B, void* C, int64_t M,
     return MB_OK;
 }
 
+size_t scratch_given(const void* workspace, size_t workspace_bytes) {
+    return workspace != nullptr ? workspace_bytes : 0;
+}
+
 // Event-timed loop shared by the mb_time_* entry points.
 template <class Launch>
 int timed_loop(Launch launch, int warmup, int iterations, hipStream_t stream, double* elapsed_s) {
@@ -362,7 +366,7 @@ size_t mb_gemm_workspace_size(int dtype, int64_t M, int64_t N, int64_t K) {
     const DeviceProps* props = nullptr;
     if (current_device_props(&props) != MB_OK) return 0;
     GemmPlan plan;
-    if (gemm_plan(dtype, M, N, K, *props, &plan) != MB_OK) return 0;
+    if (gemm_plan(dtype, M, N, K, *props, SIZE_MAX, &plan) != MB_OK) return 0;
     return plan.workspace;
 }
 
@@ -373,7 +377,7 @@ int mb_gemm(int dtype, const void* A, const void* B, void* C, int64_t M, int64_t
     int rc = device_for_launch(&props);
     if (rc != MB_OK) return rc;
     GemmPlan plan;
-    if ((rc = gemm_plan(dtype, M, N, K, *props, &plan)) != MB_OK) return rc;
+    if ((rc = gemm_plan(dtype, M, N, K, *props, scratch_given(workspace, workspace_bytes), &plan)) != MB_OK) return rc;
     if ((rc = check_gemm_args(dtype, A, B, C, M, N, K, workspace, workspace_bytes, plan)) != MB_OK)
         return rc;
     return gemm_launch(dtype, A, B, C, M, N, K, scale_a, scale_b, workspace, plan,
@@ -387,7 +391,8 @@ int mb_gemm_noalloc(int dtype, const void* A, const void* B, void* C, int64_t M,
     int rc = device_for_launch(&props);
     if (rc != MB_OK) return rc;
     GemmPlan plan;
-    if ((rc = gemm_plan(dtype, M, N, K, *props, &plan)) != MB_OK) return rc;
+    // No scratch for plans that can do without: those calls may overlap on one GPU.
+    if ((rc = gemm_plan(dtype, M, N, K, *props, 0, &plan)) != MB_OK) return rc;
     if (plan.workspace > (size_t)MB_NOALLOC_SCRATCH_BYTES) {
         set_error("GEMM %s %lldx%lldx%lld needs %zu scratch bytes; mb_gemm_noalloc holds %zu "
                   "(use mb_gemm with a caller workspace)",
@@ -409,7 +414,7 @@ int mb_time_gemm(int dtype, const void* A, const void* B, void* C, int64_t M, in
     int rc = device_for_launch(&props);
     if (rc != MB_OK) return rc;
     GemmPlan plan;
-    if ((rc = gemm_plan(dtype, M, N, K, *props, &plan)) != MB_OK) return rc;
+    if ((rc = gemm_plan(dtype, M, N, K, *props, scratch_given(workspace, workspace_bytes), &plan)) != MB_OK) return rc;
     if ((rc = check_gemm_args(dtype, A, B, C, M, N, K, workspace, workspace_bytes, plan)) != MB_OK)
         return rc;
     hipStream_t st = static_cast<hipStream_t>(stream);
@@ -432,7 +437,7 @@ int mb_time_gemm_rotating(int dtype, const void* const* A, const void* const* B,
     int rc = device_for_launch(&props);
     if (rc != MB_OK) return rc;
     GemmPlan plan;
-    if ((rc = gemm_plan(dtype, M, N, K, *props, &plan)) != MB_OK) return rc;
+    if ((rc = gemm_plan(dtype, M, N, K, *props, scratch_given(workspace, workspace_bytes), &plan)) != MB_OK) return rc;
     for (int i = 0; i < sets; ++i)
         if ((rc = check_gemm_args(dtype, A[i], B[i], C[i], M, N, K, workspace, workspace_bytes, plan)) != MB_OK)
             return rc;
@@ -475,7 +480,7 @@ int mb_kernel_info(int kind, int a, int b, int64_t m, int64_t n, int64_t k, char
     }
     if (kind == MB_KIND_GEMM) {
         GemmPlan plan;
-        if ((rc = gemm_plan(a, m, n, k, *props, &plan)) != MB_OK) return rc;
+        if ((rc = gemm_plan(a, m, n, k, *props, SIZE_MAX, &plan)) != MB_OK) return rc;
         j.str("implementation", plan.implementation);
         j.num("threads_per_block", plan.threads);
         j.num("grid_blocks", plan.grid);

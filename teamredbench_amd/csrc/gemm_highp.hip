@@ -3,13 +3,12 @@
 // accumulated in that type by the MFMAs (fp32: v_mfma_f32_32x32x2_f32; fp64:
 // v_mfma_f64_16x16x4_f64), for any M, N, K >= 1.
 //
-// Two kernels. Shapes whose A and B rows start on 16 bytes run on an LDS-DMA
-// ring like the 16-bit pipelined kernel (gemm_f32_dma_kernel,
-// gemm_f64_dma_kernel below: 95% and 93% of peak at 8192^3): fp64 on 128 x 128
-// tiles, fp32 on 256 x 256 tiles where their rounds fill the CUs and on
-// 128 x 128 tiles elsewhere (highp_dma_config). Every other shape runs the
-// register-staged kernel that follows, which takes any shape and stays near
-// 80% of peak:
+// Two kernels. An LDS-DMA ring like the 16-bit pipelined kernel
+// (gemm_f32_dma_kernel, gemm_f64_dma_kernel below: 95% and 93% of peak at
+// 8192^3) runs every shape within 32-bit buffer offsets, on tiles from 256 x
+// 256 (fp32) to 32 x 128, with K split over idle CUs when the caller gives a
+// workspace (highp_choose). The rest run the register-staged kernel that
+// follows, which indexes with 64 bits and stays near 80% of peak:
 //
 // Register-staged kernel. Operands come through registers into a
 // double-buffered LDS tile (one barrier per stage), and the next stage's
@@ -31,7 +30,6 @@
 // are skipped, so ragged edges need no separate kernel.
 #include "gemm_pipeline.hpp"
 
-#include <cstdlib>
 #include <utility>
 
 namespace mb {
@@ -234,26 +232,63 @@ gemm_highp_kernel(const T* __restrict__ A, const T* __restrict__ B, T* __restric
 // fragment hold one C row, 4 runs of 4 consecutive columns; the epilogue
 // stores them as 16-byte pieces straight from registers (a tile computes for
 // milliseconds; its 256 KiB of C do not need LDS staging).
-constexpr int kF32Stages = 4, kF32StageK = 16, kF32GroupM = 4;
+constexpr int kHpStages = 4, kHpGroupM = 4;   // ring slots; tile rows per XCD group
 
-__device__ __forceinline__ int swz_b32(int row) { return ((row >> 3) & 1) << 3; }
+// Chunk c of B row r sits at chunk c ^ swz_b32(r). Rows of 32 columns (128
+// bytes) have no chunk 8; there rows 8..15 are swapped in pairs instead
+// (f32_b_row), so that the halves' rows, 8 apart, differ in parity: the odd
+// row lies on the other half of the banks.
+template <int BN, int SK>
+__device__ __forceinline__ int swz_b32(int row) { return BN >= 64 ? (row >= SK / 2 ? 8 : 0) : 0; }
+template <int BN, int SK>
+__device__ __forceinline__ int f32_b_row(int row) { return BN >= 64 ? row : row ^ (row >= SK / 2 ? 1 : 0); }
 
-template <int BM, int BN, bool RAGGED_K = false>
-__global__ void __launch_bounds__(256)
+// A rows of 64 or 128 bytes.
+template <int ROW>
+__device__ __forceinline__ int swz_hp_a(int row) { return ROW == 64 ? swz_a(row) : swz_a2(row); }
+
+typedef f32x4 f32x4_any __attribute__((aligned(4)));
+
+// The loads that go out after MFMA s of `mfmas`: load l follows MFMA
+// l * mfmas / loads; the first such l at or after MFMA s.
+constexpr int load_at(int s, int mfmas, int loads) { return (s * loads + mfmas - 1) / mfmas; }
+
+template <int LO, int HI, class F>
+__device__ __forceinline__ void issue_range(F f) {
+    [&]<int... I>(std::integer_sequence<int, I...>) {
+        (f(std::integral_constant<int, LO + I>{}), ...);
+    }(std::make_integer_sequence<int, HI - LO>{});
+}
+
+// Tile shapes. Waves form a WGM x WGN grid of 32 x 32 fragments; a stage is SK
+// K values, 64 or 128 bytes of an A row. 128 x 128 tiles run eight waves, two
+// per SIMD, so one's barrier waits hide under the other's MFMAs (2048^3 fp32
+// 127.7 us against 137.9 with four; 4% over 335 shapes of one block per CU).
+// DMA pieces are PA / PB bytes of A / B per lane: 16, or 4 for rows off 16
+// bytes (K or N not a multiple of 4), where a lane's 16 bytes would not start
+// on 16 in memory. A 4-byte piece costs four times the load instructions,
+// which the 64-cycle MFMAs cover: fp32 4096 x 4001 x 4096 951 us against 929 at
+// N = 4096 (1659 on the register-staged kernel).
+template <int BM, int BN, int WGM, int WGN, int SK, int PA, int PB, bool RAGGED_K>
+__global__ void __launch_bounds__(64 * WGM * WGN)
 gemm_f32_dma_kernel(const float* __restrict__ A, const float* __restrict__ B, float* __restrict__ C, int M, int N,
-                    int K, int tiles_m, int tiles_n) {
-    // Per-tile sizes: waves in a 2 x 2 grid, fragments of 32 x 32.
-    constexpr int WTM = BM / 2, WTN = BN / 2, FM = WTM / 32, FN = WTN / 32;
-    constexpr int ABytes = BM * 64, BRow = BN * 4, BBytes = kF32StageK * BRow, Slot = ABytes + BBytes;
-    constexpr int AInstr = ABytes / 1024 / 4, BInstr = BBytes / 1024 / 4, Loads = AInstr + BInstr;
-    static_assert(AInstr >= 1 && BInstr >= 1 && WTM % 32 == 0 && WTN % 32 == 0 && BRow >= 256, "tile shape");
-    __shared__ __attribute__((aligned(1024))) unsigned char ring[kF32Stages][Slot];
+                    int K, int tiles_m, int tiles_n, int splits, int k_len, float* __restrict__ ws) {
+    constexpr int W = WGM * WGN;
+    constexpr int WTM = BM / WGM, WTN = BN / WGN, FM = WTM / 32, FN = WTN / 32;
+    constexpr int ARow = SK * 4, ABytes = BM * ARow, BRow = BN * 4, BBytes = SK * BRow, Slot = ABytes + BBytes;
+    constexpr int AInstr = ABytes / (64 * PA) / W, BInstr = BBytes / (64 * PB) / W, Loads = AInstr + BInstr;
+    static_assert(AInstr * W * 64 * PA == ABytes && BInstr * W * 64 * PB == BBytes, "a stage splits over the waves");
+    static_assert(WTM % 32 == 0 && WTN % 32 == 0 && BRow >= 128, "tile shape");
+    __shared__ __attribute__((aligned(1024))) unsigned char ring[kHpStages][Slot];
     const int tid = threadIdx.x, lane = tid & 63, half = lane >> 5;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int wm = wave >> 1, wn = wave & 1;
+    const int wm = wave / WGN, wn = wave % WGN;
+    const int split = splits > 1 ? (int)blockIdx.x % splits : 0;   // the splits of a tile are adjacent
+    const int tile = splits > 1 ? (int)blockIdx.x / splits : (int)blockIdx.x;
     int tm, tn;
-    tile_coords((int)blockIdx.x, tiles_m * tiles_n, tiles_m, tiles_n, kF32GroupM, &tm, &tn);
+    tile_coords(tile, tiles_m * tiles_n, tiles_m, tiles_n, kHpGroupM, &tm, &tn);
     const int lda = K * 4, ldb = N * 4;
+    const int k0 = split * k_len;
     // Buffer ranges end at A's row M and at B's last byte: rows of a partial
     // last M tile, and B's rows past K, load zeros; the columns of a partial
     // last N tile load the start of B's next row and are not stored.
@@ -264,28 +299,30 @@ gemm_f32_dma_kernel(const float* __restrict__ A, const float* __restrict__ B, fl
     int a_voff[AInstr], a_kbyte[AInstr], b_voff[BInstr];
 #pragma unroll
     for (int q = 0; q < AInstr; ++q) {
-        const int lin = (wave * AInstr + q) * 1024 + lane * 16;
-        const int row = lin / 64, pchunk = (lin % 64) >> 4;
-        a_kbyte[q] = (pchunk ^ swz_a(row)) << 4;
+        const int lin = (wave * AInstr + q) * 64 * PA + lane * PA;
+        const int row = lin / ARow, pchunk = (lin % ARow) >> 4;
+        a_kbyte[q] = ((pchunk ^ swz_hp_a<ARow>(row)) << 4) + (lin & 15);
         a_voff[q] = row * lda + a_kbyte[q];
     }
 #pragma unroll
     for (int q = 0; q < BInstr; ++q) {
-        const int lin = (wave * BInstr + q) * 1024 + lane * 16;
-        const int row = lin / BRow, pchunk = (lin % BRow) >> 4;
-        b_voff[q] = row * ldb + ((pchunk ^ swz_b32(row)) << 4);
+        const int lin = (wave * BInstr + q) * 64 * PB + lane * PB;
+        const int slot_row = lin / BRow, pchunk = (lin % BRow) >> 4;
+        b_voff[q] = f32_b_row<BN, SK>(slot_row) * ldb + ((pchunk ^ swz_b32<BN, SK>(slot_row)) << 4) + (lin & 15);
     }
     // DMA instruction q of stage kt into `slot`: A pieces first, then B.
-    // RAGGED_K (K not a multiple of the stage): A pieces at or past K load zeros.
+    // RAGGED_K (the splits' stages run past K): A pieces at or past K load zeros.
     auto issue_one = [&](int kt, int slot, auto idx) {
         constexpr int q = decltype(idx)::value;
         const unsigned base = (unsigned)(uintptr_t)(MB_LDS unsigned char*)ring[slot];
-        if constexpr (q < AInstr)
-            lds_dma16(ra, base + (wave * AInstr + q) * 1024,
-                      RAGGED_K && a_kbyte[q] >= K * 4 - kt * 64 ? (int)0x80000000u : a_voff[q], kt * 64);
-        else
-            lds_dma16(rb, base + ABytes + (wave * BInstr + q - AInstr) * 1024, b_voff[q - AInstr],
-                      kt * kF32StageK * ldb);
+        const int kb = k0 * 4 + kt * ARow;
+        if constexpr (q < AInstr) {
+            lds_dma<PA>(ra, base + (wave * AInstr + q) * 64 * PA,
+                            RAGGED_K && a_kbyte[q] >= K * 4 - kb ? (int)0x80000000u : a_voff[q], kb);
+        } else {
+            lds_dma<PB>(rb, base + ABytes + (wave * BInstr + q - AInstr) * 64 * PB, b_voff[q - AInstr],
+                        (k0 + kt * SK) * ldb);
+        }
     };
     auto issue = [&](int kt, int slot) {
         [&]<int... Q>(std::integer_sequence<int, Q...>) {
@@ -301,39 +338,43 @@ gemm_f32_dma_kernel(const float* __restrict__ A, const float* __restrict__ B, fl
 #pragma unroll
             for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
 
-    const int ksteps = (K + kF32StageK - 1) / kF32StageK, last = ksteps - 1;
+    const int ksteps = k_len / SK, last = ksteps - 1;
 #pragma unroll
-    for (int st = 0; st < kF32Stages - 1; ++st) issue(min(st, last), st);
+    for (int st = 0; st < kHpStages - 1; ++st) issue(min(st, last), st);
     const int a_row = wm * WTM + (lane & 31);
     const int b_col = wn * WTN + (lane & 31);
-    // A operands: a[i][t] is K 8h + t of fragment i's row. Steps 0-3 use the
-    // first 16-byte chunk, steps 4-7 the second, so the next stage's first
-    // chunk is read into the registers steps 0-3 are done with (after the
-    // mid-stage barrier) and its second chunk at the stage boundary, four
-    // steps before it is needed: one register set.
-    float a[FM][8];
+    // A operands: a[i][t] is K SK / 2 * h + t of fragment i's row. The next
+    // stage's first half is read into the registers this stage's first half of
+    // steps is done with (after the mid-stage barrier), its second half at the
+    // stage boundary, half a stage before it is needed: one register set.
+    float a[FM][SK / 2];
     float b[4][FN];     // B operands of steps t .. t + 3, read two steps ahead
-    auto read_a = [&](int kt, int e) {
-        const unsigned char* slot = ring[kt % kF32Stages];
+    auto read_a = [&](int kt, auto hc) {
+        constexpr int hf = decltype(hc)::value;
+        const unsigned char* slot = ring[kt % kHpStages];
 #pragma unroll
         for (int i = 0; i < FM; ++i) {
             const int row = a_row + 32 * i;
-            // Whole float vectors: __builtin_bit_cast of a single ext_vector
-            // element (bit_cast(float, v[w]) on a u32x4) is miscompiled by this
-            // clang -- it reuses element 0 and drops the other loads.
-            const f32x4 v = *reinterpret_cast<const f32x4*>(slot + row * 64 + (((2 * half + e) ^ swz_a(row)) << 4));
 #pragma unroll
-            for (int w = 0; w < 4; ++w) a[i][4 * e + w] = v[w];
+            for (int e = hf * (SK / 16); e < (hf + 1) * (SK / 16); ++e) {
+                // Whole float vectors: __builtin_bit_cast of a single ext_vector
+                // element (bit_cast(float, v[w]) on a u32x4) is miscompiled by this
+                // clang -- it reuses element 0 and drops the other loads.
+                const f32x4 v = *reinterpret_cast<const f32x4*>(
+                    slot + row * ARow + (((SK / 8 * half + e) ^ swz_hp_a<ARow>(row)) << 4));
+#pragma unroll
+                for (int w = 0; w < 4; ++w) a[i][4 * e + w] = v[w];
+            }
         }
     };
     auto read_b = [&](int kt, int t, int set) {
-        const unsigned char* sb = ring[kt % kF32Stages] + ABytes;
-        const int row = 8 * half + t;
+        const unsigned char* sb = ring[kt % kHpStages] + ABytes;
+        const int row = f32_b_row<BN, SK>(SK / 2 * half + t);
 #pragma unroll
         for (int j = 0; j < FN; ++j) {
             const int col = b_col + 32 * j;
-            b[set][j] =
-                *reinterpret_cast<const float*>(sb + row * BRow + (((col >> 2) ^ swz_b32(row)) << 4) + 4 * (col & 3));
+            b[set][j] = *reinterpret_cast<const float*>(sb + row * BRow + (((col >> 2) ^ swz_b32<BN, SK>(row)) << 4) +
+                                                        4 * (col & 3));
         }
     };
     // One barrier per stage, at its middle: it certifies that stage kt + 1 has
@@ -349,26 +390,24 @@ gemm_f32_dma_kernel(const float* __restrict__ A, const float* __restrict__ B, fl
     // latency when two blocks share a CU (3072 x 6144 x 4096 ran 17% faster
     // with two; other shapes within 0.7%). Past the last stage the loads
     // repeat it (in bounds, never used).
-    constexpr int kSteps = kF32StageK / 2, kMid = kSteps / 2;
+    constexpr int kSteps = SK / 2, kMid = kSteps / 2;
     static_assert(kSteps % 4 == 0 && kMid >= 2, "B sets cycle with the stage; next-stage reads follow the barrier");
     constexpr int kMfma = FM * FN;                               // MFMAs per step
-    constexpr int kLoadSteps = kSteps - kMid;
-    static_assert(Loads % kLoadSteps == 0 && kMfma % (Loads / kLoadSteps) == 0, "loads spread evenly");
-    constexpr int kLoadsPerStep = Loads / kLoadSteps, kLoadGap = kMfma / kLoadsPerStep;
-    wait_vmcnt_and_barrier<Loads * (kF32Stages - 2)>();
-    read_a(0, 0);
-    read_a(0, 1);
+    constexpr int kLoadMfma = kMfma * (kSteps - kMid);           // MFMAs of the second half
+    wait_vmcnt_and_barrier<Loads * (kHpStages - 2)>();
+    read_a(0, std::integral_constant<int, 0>{});
+    read_a(0, std::integral_constant<int, 1>{});
     read_b(0, 0, 0);
     read_b(0, 1, 1);
     for (int kt = 0; kt < ksteps; ++kt) {
-        const int load_kt = min(kt + kF32Stages - 1, last), load_slot = (kt + kF32Stages - 1) % kF32Stages;
+        const int load_kt = min(kt + kHpStages - 1, last), load_slot = (kt + kHpStages - 1) % kHpStages;
         [&]<int... T>(std::integer_sequence<int, T...>) {
             ([&] {
                 constexpr int t = T;
-                if (t == 0 && kt > 0) read_a(kt, 1);
+                if (t == 0 && kt > 0) read_a(kt, std::integral_constant<int, 1>{});
                 if constexpr (t == kMid) {
-                    wait_vmcnt_and_barrier<Loads * (kF32Stages - 3)>();
-                    read_a(kt + 1, 0);
+                    wait_vmcnt_and_barrier<Loads * (kHpStages - 3)>();
+                    read_a(kt + 1, std::integral_constant<int, 0>{});
                 }
                 // (t + 2) & 3 is also the set of step t + 2 - kSteps of the next stage: kSteps % 4 == 0
                 if constexpr (t + 2 < kSteps) read_b(kt, t + 2, (t + 2) & 3);
@@ -378,9 +417,11 @@ gemm_f32_dma_kernel(const float* __restrict__ A, const float* __restrict__ B, fl
                     ([&] {
                         constexpr int m = Q, i = m / FN, j = m % FN;
                         acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(b[t & 3][j], a[i][t], acc[i][j], 0, 0, 0);
-                        if constexpr (t >= kMid && m % kLoadGap == 0)
-                            issue_one(load_kt, load_slot,
-                                      std::integral_constant<int, (t - kMid) * kLoadsPerStep + m / kLoadGap>{});
+                        // Load l follows MFMA l * kLoadMfma / Loads of the second half.
+                        if constexpr (t >= kMid)
+                            issue_range<load_at((t - kMid) * kMfma + m, kLoadMfma, Loads),
+                                        load_at((t - kMid) * kMfma + m + 1, kLoadMfma, Loads)>(
+                                [&](auto idx) { issue_one(load_kt, load_slot, idx); });
                         __builtin_amdgcn_sched_barrier(0);   // keeps each load where it is placed
                     }(), ...);
                 }(std::make_integer_sequence<int, kMfma>{});
@@ -390,20 +431,32 @@ gemm_f32_dma_kernel(const float* __restrict__ A, const float* __restrict__ B, fl
     wait_vmcnt_and_barrier<0>();
 
     // Accumulator register 4g + q of lane l holds C[row 32i + l % 32]
-    // [col 32j + 8g + 4 * (l / 32) + q] of the wave's tile.
-    // Rows at or past M and 4-column groups at or past N (a multiple of 4) are not stored.
+    // [col 32j + 8g + 4 * (l / 32) + q] of the wave's tile. Rows at or past M
+    // and columns at or past N are not stored; with K splits the block stores
+    // its partial plane ws[split][M][N] instead of C.
+    float* out = splits > 1 ? ws + (int64_t)split * M * N : C;
     const int col0 = tn * BN + wn * WTN + 4 * half;
 #pragma unroll
     for (int i = 0; i < FM; ++i) {
         const int row = tm * BM + wm * WTM + 32 * i + (lane & 31);
         if (row >= M) continue;
-        float* crow = C + (int64_t)row * N + col0;
+        float* crow = out + (int64_t)row * N + col0;
 #pragma unroll
         for (int j = 0; j < FN; ++j)
 #pragma unroll
             for (int g = 0; g < 4; ++g) {
                 const f32x4 v = {acc[i][j][4 * g], acc[i][j][4 * g + 1], acc[i][j][4 * g + 2], acc[i][j][4 * g + 3]};
-                if (col0 + 32 * j + 8 * g < N) *reinterpret_cast<f32x4*>(crow + 32 * j + 8 * g) = v;
+                const int left = N - (col0 + 32 * j + 8 * g);   // columns of C from here on
+                float* p = crow + 32 * j + 8 * g;
+                if constexpr (PB == 16) {
+                    if (left > 0) *reinterpret_cast<f32x4*>(p) = v;   // N is a multiple of 4
+                } else if (left >= 4) {
+                    *reinterpret_cast<f32x4_any*>(p) = v;
+                } else {
+#pragma unroll
+                    for (int e = 0; e < 3; ++e)
+                        if (e < left) p[e] = v[e];
+                }
             }
     }
 }
@@ -426,26 +479,30 @@ gemm_f32_dma_kernel(const float* __restrict__ A, const float* __restrict__ B, fl
 // 256 x 128 tiles (one block per CU) on 12 shapes from 3072 x 6144 x 4096 to
 // 10240^2 x 4096, 8192^3 included (73.3 against 72.1 TFLOP/s), and 0.5%
 // slower on one (4608^3).
-constexpr int kF64Stages = 4, kF64StageK = 8;
+template <int SK>
+__device__ __forceinline__ int swz_b64(int row) { return ((row / (SK / 4)) & 1) << 3; }
 
-__device__ __forceinline__ int swz_b64(int row) { return ((row >> 1) & 1) << 3; }
-
-template <int BM, int BN, bool RAGGED_K = false>
-__global__ void __launch_bounds__(256)
+template <int BM, int BN, int WGM, int WGN, int SK, int PA, int PB, bool RAGGED_K>
+__global__ void __launch_bounds__(64 * WGM * WGN)
 gemm_f64_dma_kernel(const double* __restrict__ A, const double* __restrict__ B, double* __restrict__ C, int M,
-                    int N, int K, int tiles_m, int tiles_n) {
-    // Per-tile sizes: waves in a 2 x 2 grid, fragments of 16 x 16.
-    constexpr int WTM = BM / 2, WTN = BN / 2, FM = WTM / 16, FN = WTN / 16;
-    constexpr int ABytes = BM * 64, BRow = BN * 8, BBytes = kF64StageK * BRow, Slot = ABytes + BBytes;
-    constexpr int AInstr = ABytes / 1024 / 4, BInstr = BBytes / 1024 / 4, Loads = AInstr + BInstr;
-    static_assert(AInstr >= 1 && BInstr >= 1 && WTM % 16 == 0 && WTN % 16 == 0 && BRow >= 256, "tile shape");
-    __shared__ __attribute__((aligned(1024))) unsigned char ring[kF64Stages][Slot];
+                    int N, int K, int tiles_m, int tiles_n, int splits, int k_len, double* __restrict__ ws) {
+    // Waves in a WGM x WGN grid of 16 x 16 fragments; pieces as in gemm_f32_dma_kernel.
+    constexpr int W = WGM * WGN;
+    constexpr int WTM = BM / WGM, WTN = BN / WGN, FM = WTM / 16, FN = WTN / 16;
+    constexpr int ARow = SK * 8, ABytes = BM * ARow, BRow = BN * 8, BBytes = SK * BRow, Slot = ABytes + BBytes;
+    constexpr int AInstr = ABytes / (64 * PA) / W, BInstr = BBytes / (64 * PB) / W, Loads = AInstr + BInstr;
+    static_assert(AInstr * W * 64 * PA == ABytes && BInstr * W * 64 * PB == BBytes, "a stage splits over the waves");
+    static_assert(WTM % 16 == 0 && WTN % 16 == 0 && BRow >= 256, "tile shape");
+    __shared__ __attribute__((aligned(1024))) unsigned char ring[kHpStages][Slot];
     const int tid = threadIdx.x, lane = tid & 63, grp = lane >> 4;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int wm = wave >> 1, wn = wave & 1;
+    const int wm = wave / WGN, wn = wave % WGN;
+    const int split = splits > 1 ? (int)blockIdx.x % splits : 0;
+    const int tile = splits > 1 ? (int)blockIdx.x / splits : (int)blockIdx.x;
     int tm, tn;
-    tile_coords((int)blockIdx.x, tiles_m * tiles_n, tiles_m, tiles_n, kF32GroupM, &tm, &tn);
+    tile_coords(tile, tiles_m * tiles_n, tiles_m, tiles_n, kHpGroupM, &tm, &tn);
     const int lda = K * 8, ldb = N * 8;
+    const int k0 = split * k_len;
     // Buffer ranges as in gemm_f32_dma_kernel: partial last tiles and a ragged K.
     const __amdgpu_buffer_rsrc_t ra = __builtin_amdgcn_make_buffer_rsrc(
         const_cast<double*>(A) + (int64_t)tm * BM * K, (short)0, min(BM, M - tm * BM) * lda, kBufferFlags);
@@ -454,26 +511,28 @@ gemm_f64_dma_kernel(const double* __restrict__ A, const double* __restrict__ B, 
     int a_voff[AInstr], a_kbyte[AInstr], b_voff[BInstr];
 #pragma unroll
     for (int q = 0; q < AInstr; ++q) {
-        const int lin = (wave * AInstr + q) * 1024 + lane * 16;
-        const int row = lin / 64, pchunk = (lin % 64) >> 4;
-        a_kbyte[q] = (pchunk ^ swz_a(row)) << 4;
+        const int lin = (wave * AInstr + q) * 64 * PA + lane * PA;
+        const int row = lin / ARow, pchunk = (lin % ARow) >> 4;
+        a_kbyte[q] = ((pchunk ^ swz_hp_a<ARow>(row)) << 4) + (lin & 15);
         a_voff[q] = row * lda + a_kbyte[q];
     }
 #pragma unroll
     for (int q = 0; q < BInstr; ++q) {
-        const int lin = (wave * BInstr + q) * 1024 + lane * 16;
+        const int lin = (wave * BInstr + q) * 64 * PB + lane * PB;
         const int row = lin / BRow, pchunk = (lin % BRow) >> 4;
-        b_voff[q] = row * ldb + ((pchunk ^ swz_b64(row)) << 4);
+        b_voff[q] = row * ldb + ((pchunk ^ swz_b64<SK>(row)) << 4) + (lin & 15);
     }
     auto issue_one = [&](int kt, int slot, auto idx) {
         constexpr int q = decltype(idx)::value;
         const unsigned base = (unsigned)(uintptr_t)(MB_LDS unsigned char*)ring[slot];
-        if constexpr (q < AInstr)
-            lds_dma16(ra, base + (wave * AInstr + q) * 1024,
-                      RAGGED_K && a_kbyte[q] >= K * 8 - kt * 64 ? (int)0x80000000u : a_voff[q], kt * 64);
-        else
-            lds_dma16(rb, base + ABytes + (wave * BInstr + q - AInstr) * 1024, b_voff[q - AInstr],
-                      kt * kF64StageK * ldb);
+        const int kb = k0 * 8 + kt * ARow;
+        if constexpr (q < AInstr) {
+            lds_dma<PA>(ra, base + (wave * AInstr + q) * 64 * PA,
+                            RAGGED_K && a_kbyte[q] >= K * 8 - kb ? (int)0x80000000u : a_voff[q], kb);
+        } else {
+            lds_dma<PB>(rb, base + ABytes + (wave * BInstr + q - AInstr) * 64 * PB, b_voff[q - AInstr],
+                        (k0 + kt * SK) * ldb);
+        }
     };
     auto issue = [&](int kt, int slot) {
         [&]<int... Q>(std::integer_sequence<int, Q...>) {
@@ -489,67 +548,72 @@ gemm_f64_dma_kernel(const double* __restrict__ A, const double* __restrict__ B, 
 #pragma unroll
             for (int r = 0; r < 4; ++r) acc[i][j][r] = 0.0;
 
-    const int ksteps = (K + kF64StageK - 1) / kF64StageK, last = ksteps - 1;
+    const int ksteps = k_len / SK, last = ksteps - 1;
 #pragma unroll
-    for (int st = 0; st < kF64Stages - 1; ++st) issue(min(st, last), st);
+    for (int st = 0; st < kHpStages - 1; ++st) issue(min(st, last), st);
     const int a_row = wm * WTM + (lane & 15);
     const int b_col = wn * WTN + (lane & 15);
-    double a[2][FM][2];  // A operands of this stage and the next
-    double b[2][FN];     // B operands of this step and the next
+    constexpr int kSteps = SK / 4, kMid = kSteps / 2;   // group g takes K kSteps * g + t at step t
+    double a[2][FM][kSteps];  // A operands of this stage and the next
+    double b[2][FN];          // B operands of this step and the next
     auto read_a = [&](int kt, auto setc) {
         constexpr int set = decltype(setc)::value;
-        const unsigned char* slot = ring[kt % kF64Stages];
+        const unsigned char* slot = ring[kt % kHpStages];
 #pragma unroll
         for (int i = 0; i < FM; ++i) {
             const int row = a_row + 16 * i;
-            const f64x2 v = *reinterpret_cast<const f64x2*>(slot + row * 64 + ((grp ^ swz_a(row)) << 4));
-            a[set][i][0] = v[0];
-            a[set][i][1] = v[1];
+#pragma unroll
+            for (int e = 0; e < kSteps / 2; ++e) {
+                const f64x2 v = *reinterpret_cast<const f64x2*>(
+                    slot + row * ARow + (((kSteps / 2 * grp + e) ^ swz_hp_a<ARow>(row)) << 4));
+                a[set][i][2 * e] = v[0];
+                a[set][i][2 * e + 1] = v[1];
+            }
         }
     };
     auto read_b = [&](int kt, int t, int set) {
-        const unsigned char* sb = ring[kt % kF64Stages] + ABytes;
-        const int row = 2 * grp + t;
+        const unsigned char* sb = ring[kt % kHpStages] + ABytes;
+        const int row = kSteps * grp + t;
 #pragma unroll
         for (int j = 0; j < FN; ++j) {
             const int col = b_col + 16 * j;
-            b[set][j] = *reinterpret_cast<const double*>(sb + row * BRow + (((col >> 1) ^ swz_b64(row)) << 4) +
+            b[set][j] = *reinterpret_cast<const double*>(sb + row * BRow + (((col >> 1) ^ swz_b64<SK>(row)) << 4) +
                                                          8 * (col & 1));
         }
     };
-    // The fp32 kernel's schedule: one barrier per stage, between its two
-    // steps, after which stage kt + 1's A operands are read under the second
-    // step's MFMAs and its first B operands at the end of the stage; stage
-    // kt + 3's loads are spread evenly between the second step's MFMAs.
-    constexpr int kMfma = FM * FN, kLoadGap = kMfma / Loads;
-    static_assert(kLoadGap >= 1, "a load per MFMA at most");
+    // The fp32 kernel's schedule: one barrier per stage, at its middle, after
+    // which stage kt + 1's A operands are read under the second half's MFMAs
+    // and its first B operands at the end of the stage; the loads of stage
+    // kt + kHpStages - 1 are spread evenly between the second half's MFMAs.
+    constexpr int kMfma = FM * FN, kLoadMfma = kMfma * (kSteps - kMid);
     auto stage = [&](int kt, auto curc) {
         constexpr int cur = decltype(curc)::value;
-        const int load_kt = min(kt + kF64Stages - 1, last), load_slot = (kt + kF64Stages - 1) % kF64Stages;
+        const int load_kt = min(kt + kHpStages - 1, last), load_slot = (kt + kHpStages - 1) % kHpStages;
         [&]<int... T>(std::integer_sequence<int, T...>) {
             ([&] {
                 constexpr int t = T;
-                if constexpr (t == 1) {
-                    wait_vmcnt_and_barrier<Loads * (kF64Stages - 3)>();
+                if constexpr (t == kMid) {
+                    wait_vmcnt_and_barrier<Loads * (kHpStages - 3)>();
                     read_a(kt + 1, std::integral_constant<int, cur ^ 1>{});
-                    read_b(kt + 1, 0, 0);
-                } else {
-                    read_b(kt, 1, 1);
                 }
+                if constexpr (t + 1 < kSteps) read_b(kt, t + 1, (t + 1) & 1);
+                else read_b(kt + 1, 0, 0);
                 __builtin_amdgcn_sched_barrier(0);
                 [&]<int... Q>(std::integer_sequence<int, Q...>) {
                     ([&] {
                         constexpr int m = Q, i = m / FN, j = m % FN;
-                        acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[cur][i][t], b[t][j], acc[i][j], 0, 0, 0);
-                        if constexpr (t == 1 && m % kLoadGap == 0 && m / kLoadGap < Loads)
-                            issue_one(load_kt, load_slot, std::integral_constant<int, m / kLoadGap>{});
+                        acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[cur][i][t], b[t & 1][j], acc[i][j], 0, 0, 0);
+                        if constexpr (t >= kMid)
+                            issue_range<load_at((t - kMid) * kMfma + m, kLoadMfma, Loads),
+                                        load_at((t - kMid) * kMfma + m + 1, kLoadMfma, Loads)>(
+                                [&](auto idx) { issue_one(load_kt, load_slot, idx); });
                         __builtin_amdgcn_sched_barrier(0);   // keeps each load where it is placed
                     }(), ...);
                 }(std::make_integer_sequence<int, kMfma>{});
             }(), ...);
-        }(std::make_integer_sequence<int, 2>{});
+        }(std::make_integer_sequence<int, kSteps>{});
     };
-    wait_vmcnt_and_barrier<Loads * (kF64Stages - 2)>();
+    wait_vmcnt_and_barrier<Loads * (kHpStages - 2)>();
     read_a(0, std::integral_constant<int, 0>{});
     read_b(0, 0, 0);
     for (int kt = 0; kt < ksteps; kt += 2) {
@@ -558,7 +622,9 @@ gemm_f64_dma_kernel(const double* __restrict__ A, const double* __restrict__ B, 
     }
     wait_vmcnt_and_barrier<0>();
 
-    // Rows at or past M and columns at or past N are not stored.
+    // Rows at or past M and columns at or past N are not stored; with K splits
+    // the block stores its partial plane.
+    double* out = splits > 1 ? ws + (int64_t)split * M * N : C;
     const int col0 = tn * BN + wn * WTN + (lane & 15);
 #pragma unroll
     for (int i = 0; i < FM; ++i)
@@ -566,54 +632,105 @@ gemm_f64_dma_kernel(const double* __restrict__ A, const double* __restrict__ B, 
         for (int r = 0; r < 4; ++r) {
             const int row = tm * BM + wm * WTM + 16 * i + 4 * r + grp;
             if (row >= M) continue;
-            double* crow = C + (int64_t)row * N + col0;
+            double* crow = out + (int64_t)row * N + col0;
 #pragma unroll
             for (int j = 0; j < FN; ++j)
                 if (col0 + 16 * j < N) crow[16 * j] = acc[i][j][r];
         }
 }
 
-// Which LDS-DMA ring a shape takes: 1 = fp32 on 256 x 256 tiles, when they
-// cover every CU and their rounds cost no more than 128 x 128 tiles' (rule
-// below); 2 = 128 x 128 tiles, every other fp32 shape and every fp64 one,
-// partial last tiles included. 0 = the register-staged kernel, with *why naming the
-// reason: A's or B's rows not on 16 bytes, or buffer offsets (B's K x N bytes,
-// a 256-row A panel) beyond 31 bits. A K that is not whole stages runs the
-// RAGGED_K instantiations, whose A pieces past K load zeros.
-int highp_dma_config(bool f64, int64_t M, int64_t N, int64_t K, int cus, const char** why) {
+// Sum of the K-split partials: C[i] = sum_s ws[s][i] over planes of `mn`
+// elements, in split order. A thread takes 16 bytes of C and has L splits'
+// loads in flight (the planes were just written: the pass is latency-bound).
+// Planes and C need only element alignment.
+template <typename T, int L>
+__global__ void __launch_bounds__(64)
+highp_split_sum_kernel(const T* __restrict__ ws, T* __restrict__ C, int64_t mn, int splits) {
+    constexpr int V = 16 / (int)sizeof(T);
+    typedef T Vec __attribute__((ext_vector_type(V)));
+    typedef Vec VecAny __attribute__((aligned(sizeof(T))));
+    const int64_t i = ((int64_t)blockIdx.x * 64 + threadIdx.x) * V;
+    if (i + V <= mn) {
+        Vec sum = *reinterpret_cast<const VecAny*>(ws + i);
+        for (int s0 = 1; s0 < splits; s0 += L) {
+            Vec v[L];
+#pragma unroll
+            for (int u = 0; u < L; ++u)
+                v[u] = s0 + u < splits ? (Vec)*reinterpret_cast<const VecAny*>(ws + (s0 + u) * mn + i) : (Vec)T(0);
+#pragma unroll
+            for (int u = 0; u < L; ++u)
+                if (s0 + u < splits) sum += v[u];
+        }
+        *reinterpret_cast<VecAny*>(C + i) = sum;
+    } else {
+        for (int64_t e = i; e < mn; ++e) {
+            T sum = ws[e];
+            for (int s = 1; s < splits; ++s) sum += ws[s * mn + e];
+            C[e] = sum;
+        }
+    }
+}
+
+// Tiles of the LDS-DMA rings, by plan->config (0: the register-staged kernel).
+struct HighpTile {
+    int bm, bn, wgm, wgn;
+    int row;                // bytes of A's K per row and stage: 64, or 128 (whole cache lines)
+};
+constexpr HighpTile kHighpTiles[] = {
+    {128, 128, 0, 0, 64},   // 0: register-staged
+    {256, 256, 2, 2, 64},   // 1: fp32 only
+    {128, 128, 4, 2, 64},   // 2
+    {128, 128, 4, 2, 128},  // 3: fp64, one block per CU
+    {64, 64, 2, 2, 64},     // 4
+    {32, 128, 1, 4, 128},   // 5
+    {128, 32, 4, 1, 128},   // 6
+};
+
+// The ring's tile and K splits for a shape, using at most `scratch` bytes of
+// partial planes; config 0 with *why set for a shape only the register-staged
+// kernel takes.
+struct HighpChoice {
+    int config = 0, splits = 1;
+    bool pieces4 = false;    // A's or B's rows off 16 bytes: 4-byte DMA pieces
+};
+
+HighpChoice highp_choose(bool f64, int64_t M, int64_t N, int64_t K, int cus, size_t scratch, const char** why) {
+    HighpChoice ch;
     if (tuning(MB_TUNE_GEMM_HIGHP_STAGED) == 1) {
         *why = "forced by the gemm_highp_staged override";
-        return 0;
+        return ch;
     }
-    const int64_t e = f64 ? 8 : 4, stage_k = f64 ? kF64StageK : kF32StageK;
-    // The DMA loads need A's and B's rows on 16 bytes.
-    if ((K * e) % 16 != 0) {
-        *why = f64 ? "K is not a multiple of 2" : "K is not a multiple of 4";
-        return 0;
-    }
-    if ((N * e) % 16 != 0) {
-        *why = f64 ? "N is not a multiple of 2" : "N is not a multiple of 4";
-        return 0;
-    }
-    const int64_t k_pad = (K + stage_k - 1) / stage_k * stage_k;
-    if ((k_pad * N + 256) * e >= (int64_t(1) << 31) || 256 * k_pad * e >= (int64_t(1) << 31)) {
+    const int64_t e = f64 ? 8 : 4;
+    // Bytes of B up to a split's last stage and a partial tile's columns, and of an A panel.
+    auto k_len = [&](int c, int64_t sp) {   // K per split, whole stages
+        const int64_t stage_k = kHighpTiles[c].row / e, stages = (K + stage_k - 1) / stage_k;
+        return (stages + sp - 1) / sp * stage_k;
+    };
+    auto fits = [&](int64_t sp) {
+        const int64_t k_end = k_len(4, sp) * sp;   // the longest stages
+        return (k_end * N + 256) * e < (int64_t(1) << 31) && 256 * k_end * e < (int64_t(1) << 31);
+    };
+    if (!fits(1)) {
         *why = "operand offsets exceed 32-bit buffer addressing (K*N or 256*K bytes >= 2 GiB)";
-        return 0;
+        return ch;
     }
     // The LDS-DMA kernels take M and N as int (row and column guards); the
     // register-staged kernel indexes with int64.
     if (M >= (int64_t(1) << 31) || N >= (int64_t(1) << 31)) {
         *why = "M or N >= 2^31 exceeds the 32-bit row and column indexes of the LDS-DMA kernels";
-        return 0;
+        return ch;
     }
-    auto tiles = [&](int64_t tm, int64_t tn) { return ((M + tm - 1) / tm) * ((N + tn - 1) / tn); };
-    auto rounds = [&](int64_t t) { return (t + cus - 1) / cus; };
-    const int64_t small = tiles(128, 128), large = tiles(256, 256);
-    if (small > INT32_MAX) {
+    auto tiles = [&](int c) {
+        return ((M + kHighpTiles[c].bm - 1) / kHighpTiles[c].bm) * ((N + kHighpTiles[c].bn - 1) / kHighpTiles[c].bn);
+    };
+    if (tiles(2) > INT32_MAX) {
         *why = "more than 2^31 tiles";
-        return 0;
+        return ch;
     }
-    if (f64) return 2;   // 128 x 128 tiles: two blocks per CU (gemm_f64_dma_kernel)
+    if ((K * e) % 16 != 0) *why = f64 ? "K is not a multiple of 2" : "K is not a multiple of 4";
+    else if ((N * e) % 16 != 0) *why = f64 ? "N is not a multiple of 2" : "N is not a multiple of 4";
+    ch.pieces4 = **why != 0;
+    auto rounds = [&](int64_t blocks) { return (blocks + cus - 1) / cus; };
     // fp32: 256 x 256 tiles run 2.5% faster per FLOP than 128 x 128 ones
     // (8192^3, whole rounds of either: 150.1 against 145.8 TFLOP/s on MI355X) but
     // come in rounds of four times the work, so they are taken only when their
@@ -622,33 +739,107 @@ int highp_dma_config(bool f64, int64_t M, int64_t N, int64_t K, int cus, const c
     // 4096^3, 8192^3, 6144 x 8192 x 4096 and 5632^2 x 4096 (1.9 rounds, 2%);
     // 128 x 128 where the last 256 x 256 round is partly empty, 1.05-1.32x
     // faster there (6144^3 124.5 against 109.5 TFLOP/s, 3072 x 6144 x 4096
-    // 109.3 against 83.9). Ragged M or N: partial last tiles on either.
-    const bool large_pays = large >= cus && 4.0 * 0.975 * (double)rounds(large) <= (double)rounds(small);
-    if (M % 256 == 0 && N % 256 == 0 && large_pays) return 1;
-    if (M % 128 == 0 && N % 128 == 0) return 2;
-    return large_pays ? 1 : 2;
-}
-
-void highp_dma_tile(int cfg, int* bm, int* bn) {
-    *bm = *bn = cfg == 1 ? 256 : 128;
-}
-
-template <typename T, int BM, int BN>
-int launch_dma(const void* A, const void* B, void* C, int64_t M, int64_t N, int64_t K, hipStream_t stream) {
-    const int tiles_m = (int)((M + BM - 1) / BM), tiles_n = (int)((N + BN - 1) / BN);
-    const T* a = static_cast<const T*>(A);
-    const T* b = static_cast<const T*>(B);
-    T* c = static_cast<T*>(C);
-    const dim3 grid(tiles_m * tiles_n);
-    if constexpr (sizeof(T) == 4) {
-        auto kernel = K % kF32StageK != 0 ? gemm_f32_dma_kernel<BM, BN, true> : gemm_f32_dma_kernel<BM, BN, false>;
-        hipLaunchKernelGGL(kernel, grid, dim3(256), 0, stream, a, b, c, (int)M, (int)N, (int)K, tiles_m, tiles_n);
-    } else {
-        auto kernel = K % kF64StageK != 0 ? gemm_f64_dma_kernel<BM, BN, true> : gemm_f64_dma_kernel<BM, BN, false>;
-        hipLaunchKernelGGL(kernel, grid, dim3(256), 0, stream, a, b, c, (int)M, (int)N, (int)K, tiles_m, tiles_n);
+    // 109.3 against 83.9). Ragged M or N: partial last tiles on either. Their
+    // 32 loads per wave and stage leave no room in vmcnt for 4-byte pieces.
+    if (!f64 && !ch.pieces4 && tiles(1) >= cus &&
+        4.0 * 0.975 * (double)rounds(tiles(1)) <= (double)rounds(tiles(2))) {
+        ch.config = 1;
+        return ch;
     }
+    // 128 x 128 tiles where they fill whole rounds exactly, and for K of a few
+    // stages, where the tile hardly matters. fp64 with one block per CU takes
+    // 128-byte rows of A (2048^3 251 against 261 us; with more blocks their
+    // 128 KiB of ring leave one block per CU and run 4-9% slower).
+    if ((M % 128 == 0 && N % 128 == 0 && tiles(2) % cus == 0) || (K < 128 && M >= 512)) {
+        ch.config = f64 && tiles(2) <= cus && K >= 128 ? 3 : 2;
+        return ch;
+    }
+    // The rest: the tile and the K split that a cost model rates fastest,
+    //   MFMA     = rounds x 2 * BM * BN * K / splits at the tile's share of a
+    //              CU's peak: 0.89 on 128 x 128 and 64 x 64 tiles, 0.97 on
+    //              32 x 128 (0.83 of that above two blocks per CU, more than
+    //              its 80 KiB of ring lets share one), and 0.89 of it for the
+    //              two small tiles alone on a CU, whose barriers nothing covers;
+    //   stream   = A's and B's bytes at 8 TB/s x the share of the CUs in use;
+    //   partials = the planes written and read at that rate, + 3.2 us;
+    //   time     = max(MFMA, stream) + rounds x 1.9 us + partials,
+    // its constants fitted to the cost of the pick over 655 shapes on MI355X (M
+    // 1..4096, N and K 512..8192, aligned and odd; every tile x split 1..32):
+    // the pick is within 1.3% of the best on average. Before, 128 x 128 tiles
+    // without a split ran them all, on as few CUs as they covered: fp32 16 x
+    // 8192 x 8192 479 us against 47, 1000 x 1500 x 2000 125 against 57,
+    // 1 x 4096 x 4096 239 against 17.5; fp64 16 x 8192 x 4096 488 against 51.
+    const double cu_rate = (f64 ? 72e6 : 150e6) / 256.0;   // FLOP per us and CU
+    constexpr double kBw = 8.0e6;                           // bytes per us
+    constexpr int kTiles[] = {2, 4, 5};
+    constexpr double kEff[] = {0.89, 0.89, 0.97};
+    constexpr int kSplits[] = {1, 2, 3, 4, 6, 8, 12, 16, 24, 32};
+    double best = -1.0;
+    for (int i = 0; i < 3; ++i) {
+        const int c = kTiles[i];
+        for (const int sp : kSplits) {
+            const int64_t blocks = tiles(c) * sp, kl = k_len(c, sp);
+            if (sp > 1 && (K < 64 * sp || kl * (sp - 1) >= K || 4 * cus < blocks || !fits(sp) ||
+                           (size_t)(sp * M * N * e) > scratch))
+                continue;
+            const double r = (double)rounds(blocks), used = blocks < cus ? (double)blocks / (double)cus : 1.0;
+            const double eff = kEff[i] * (c != 2 && blocks <= cus ? 0.89 : c == 5 && blocks > 2 * cus ? 0.83 : 1.0);
+            const double mfma = r * 2.0 * kHighpTiles[c].bm * kHighpTiles[c].bn * (double)kl / (cu_rate * eff);
+            const double stream = (double)((M * K + K * N) * e) / (kBw * used);
+            const double partials = sp > 1 ? 2.0 * (double)(sp * M * N * e) / kBw + 3.2 : 0.0;
+            const double t = (mfma > stream ? mfma : stream) + r * 1.9 + partials;
+            if (best < 0.0 || t < best) best = t, ch.config = c, ch.splits = sp;
+        }
+    }
+    // One unsplit round of at least six 128-row panels runs 128 x 32 tiles:
+    // 128-row tiles without a workspace are what a plan of 1000^3 has always
+    // reported (26.7 us fp32 and 41.9 fp64, against 65 and 123 on 128 x 128;
+    // 64 x 64 tiles take 21.8 and 39.0).
+    if (ch.splits == 1 && ch.config != 2 && M >= 768 && tiles(4) <= cus) ch.config = 6;
+    return ch;
+}
+
+template <typename T, int CFG, bool PIECES4>
+int launch_dma(const void* A, const void* B, void* C, int64_t M, int64_t N, int64_t K, const GemmPlan& plan,
+               void* workspace, hipStream_t stream) {
+    constexpr HighpTile t = kHighpTiles[CFG];
+    constexpr int PA = PIECES4 ? 4 : 16, PB = PA;
+    const int tiles_m = (int)((M + t.bm - 1) / t.bm), tiles_n = (int)((N + t.bn - 1) / t.bn);
+    const int splits = plan.split_k;
+    constexpr int SK = t.row / (int)sizeof(T);
+    const int64_t stages = (K + SK - 1) / SK;
+    const int64_t k_len = (stages + splits - 1) / splits * SK;
+    T* c = static_cast<T*>(C);
+    T* ws = splits > 1 ? static_cast<T*>(workspace) : nullptr;
+    typedef void (*Kernel)(const T*, const T*, T*, int, int, int, int, int, int, int, T*);
+    Kernel kernel;
+    const bool ragged = k_len * splits != K;
+    if constexpr (sizeof(T) == 4)
+        kernel = ragged ? gemm_f32_dma_kernel<t.bm, t.bn, t.wgm, t.wgn, SK, PA, PB, true>
+                        : gemm_f32_dma_kernel<t.bm, t.bn, t.wgm, t.wgn, SK, PA, PB, false>;
+    else
+        kernel = ragged ? gemm_f64_dma_kernel<t.bm, t.bn, t.wgm, t.wgn, SK, PA, PB, true>
+                        : gemm_f64_dma_kernel<t.bm, t.bn, t.wgm, t.wgn, SK, PA, PB, false>;
+    hipLaunchKernelGGL(kernel, dim3((unsigned)(tiles_m * tiles_n * splits)), dim3(64 * t.wgm * t.wgn), 0, stream,
+                       static_cast<const T*>(A), static_cast<const T*>(B), c, (int)M, (int)N, (int)K, tiles_m, tiles_n,
+                       splits, (int)k_len, ws);
     MB_HIP_TRY(hipGetLastError());
+    if (splits > 1) {
+        const int64_t mn = M * N, per_block = 64 * (16 / (int64_t)sizeof(T));
+        auto sum = splits <= 5 ? highp_split_sum_kernel<T, 4> : highp_split_sum_kernel<T, 16>;
+        hipLaunchKernelGGL(sum, dim3((unsigned)((mn + per_block - 1) / per_block)), dim3(64), 0, stream,
+                           static_cast<const T*>(ws), c, mn, splits);
+        MB_HIP_TRY(hipGetLastError());
+    }
     return MB_OK;
+}
+
+template <typename T, int CFG>
+int launch_pieces(const void* A, const void* B, void* C, int64_t M, int64_t N, int64_t K, const GemmPlan& plan,
+                  void* workspace, hipStream_t stream) {
+    constexpr int64_t V = 16 / (int64_t)sizeof(T);
+    if (K % V == 0 && N % V == 0) return launch_dma<T, CFG, false>(A, B, C, M, N, K, plan, workspace, stream);
+    return launch_dma<T, CFG, true>(A, B, C, M, N, K, plan, workspace, stream);
 }
 
 template <typename T>
@@ -669,30 +860,34 @@ int launch_typed(const void* A, const void* B, void* C, int64_t M, int64_t N, in
 
 }  // namespace
 
-int gemm_highp_plan(int dtype, int64_t M, int64_t N, int64_t K, const DeviceProps& props, GemmPlan* plan) {
+int gemm_highp_plan(int dtype, int64_t M, int64_t N, int64_t K, const DeviceProps& props, size_t scratch,
+                    GemmPlan* plan) {
     const bool f64 = dtype == MB_DT_FLOAT64;
     const char* why = "";
-    const int cfg = highp_dma_config(f64, M, N, K, props.cu_count > 0 ? props.cu_count : 256, &why);
-    if (cfg != 0) {
-        int bm, bn;
-        highp_dma_tile(cfg, &bm, &bn);
-        plan->implementation = f64 ? "gfx950_mfma_f64_16x16x4_lds_dma" : "gfx950_mfma_f32_32x32x2_lds_dma";
-        plan->threads = 256;
-        plan->grid = (int)(((M + bm - 1) / bm) * ((N + bn - 1) / bn));
-        plan->tile_m = bm;
-        plan->tile_n = bn;
-        plan->tile_k = f64 ? kF64StageK : kF32StageK;
-        plan->wave_grid_m = plan->wave_grid_n = 2;
-        plan->frag_m = plan->frag_n = f64 ? 16 : 32;
-        plan->frag_k = f64 ? 4 : 2;
-        plan->wave_tile_m = bm / 2 / plan->frag_m;
-        plan->wave_tile_n = bn / 2 / plan->frag_n;
-        plan->k_stages = f64 ? kF64Stages : kF32Stages;
-        plan->split_k = 1;
-        plan->tile_group_m = kF32GroupM;
-        plan->workspace = 0;
-        plan->variant = kVariantHighp;
-        plan->config = cfg;
+    const HighpChoice ch = highp_choose(f64, M, N, K, props.cu_count > 0 ? props.cu_count : 256, scratch, &why);
+    plan->variant = kVariantHighp;
+    plan->config = ch.config;
+    plan->fallback = why;
+    plan->frag_m = plan->frag_n = f64 ? 16 : 32;
+    plan->frag_k = f64 ? 4 : 2;
+    const HighpTile& t = kHighpTiles[ch.config];
+    plan->tile_k = t.row / (f64 ? 8 : 4);
+    plan->tile_m = t.bm;
+    plan->tile_n = t.bn;
+    if (ch.config != 0) {
+        // The plain name when the rows are off 16 bytes: `fallback` then says why 16-byte pieces do not reach.
+        plan->implementation = f64 ? (ch.pieces4 ? "gfx950_mfma_f64_16x16x4" : "gfx950_mfma_f64_16x16x4_lds_dma")
+                                   : (ch.pieces4 ? "gfx950_mfma_f32_32x32x2" : "gfx950_mfma_f32_32x32x2_lds_dma");
+        plan->threads = 64 * t.wgm * t.wgn;
+        plan->grid = (int)(((M + t.bm - 1) / t.bm) * ((N + t.bn - 1) / t.bn) * ch.splits);
+        plan->wave_grid_m = t.wgm;
+        plan->wave_grid_n = t.wgn;
+        plan->wave_tile_m = t.bm / t.wgm / plan->frag_m;
+        plan->wave_tile_n = t.bn / t.wgn / plan->frag_n;
+        plan->k_stages = f64 ? kHpStages : kHpStages;
+        plan->split_k = ch.splits;
+        plan->tile_group_m = kHpGroupM;
+        plan->workspace = ch.splits > 1 ? (size_t)ch.splits * (size_t)M * (size_t)N * (f64 ? 8 : 4) : 0;
         return MB_OK;
     }
     const int64_t gx = (N + kHpBN - 1) / kHpBN, gy = (M + kHpBM - 1) / kHpBM;
@@ -704,37 +899,38 @@ int gemm_highp_plan(int dtype, int64_t M, int64_t N, int64_t K, const DeviceProp
     plan->implementation = f64 ? "gfx950_mfma_f64_16x16x4" : "gfx950_mfma_f32_32x32x2";
     plan->threads = kHpThreads;
     plan->grid = (int)(gx * gy);
-    plan->tile_m = kHpBM;
-    plan->tile_n = kHpBN;
-    plan->tile_k = f64 ? HighpTraits<double>::kBK : HighpTraits<float>::kBK;
     plan->wave_grid_m = 2;
     plan->wave_grid_n = 2;
-    plan->frag_m = plan->frag_n = f64 ? 16 : 32;
-    plan->frag_k = f64 ? 4 : 2;
     plan->wave_tile_m = plan->wave_tile_n = 64 / plan->frag_m;
     plan->k_stages = 2;
     plan->split_k = 1;
     plan->tile_group_m = 1;
     plan->workspace = 0;
-    plan->fallback = why;
-    plan->variant = kVariantHighp;
     return MB_OK;
 }
 
 int gemm_highp_launch(int dtype, const void* A, const void* B, void* C, int64_t M, int64_t N, int64_t K,
-                      const GemmPlan& plan, hipStream_t stream) {
-    switch (dtype) {
-        case MB_DT_FLOAT32:
-            if (plan.config == 1) return launch_dma<float, 256, 256>(A, B, C, M, N, K, stream);
-            if (plan.config == 2) return launch_dma<float, 128, 128>(A, B, C, M, N, K, stream);
-            return launch_typed<float>(A, B, C, M, N, K, stream);
-        case MB_DT_FLOAT64:
-            if (plan.config == 2) return launch_dma<double, 128, 128>(A, B, C, M, N, K, stream);
-            return launch_typed<double>(A, B, C, M, N, K, stream);
-        default:
-            set_error("fp32/fp64 GEMM: unsupported dtype %d", dtype);
-            return MB_ERR_UNSUPPORTED;
-    }
+                      const GemmPlan& plan, void* workspace, hipStream_t stream) {
+    auto run = [&](auto zero) -> int {
+        typedef decltype(zero) T;
+        switch (plan.config) {
+            case 1:
+                if constexpr (sizeof(T) == 4) return launch_dma<T, 1, false>(A, B, C, M, N, K, plan, workspace, stream);
+                break;
+            case 2: return launch_pieces<T, 2>(A, B, C, M, N, K, plan, workspace, stream);
+            case 3:
+                if constexpr (sizeof(T) == 8) return launch_pieces<T, 3>(A, B, C, M, N, K, plan, workspace, stream);
+                break;
+            case 4: return launch_pieces<T, 4>(A, B, C, M, N, K, plan, workspace, stream);
+            case 5: return launch_pieces<T, 5>(A, B, C, M, N, K, plan, workspace, stream);
+            case 6: return launch_pieces<T, 6>(A, B, C, M, N, K, plan, workspace, stream);
+        }
+        return launch_typed<T>(A, B, C, M, N, K, stream);
+    };
+    if (dtype == MB_DT_FLOAT32) return run(0.0f);
+    if (dtype == MB_DT_FLOAT64) return run(0.0);
+    set_error("fp32/fp64 GEMM: unsupported dtype %d", dtype);
+    return MB_ERR_UNSUPPORTED;
 }
 
 }  // namespace mb

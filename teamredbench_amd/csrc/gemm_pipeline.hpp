@@ -18,6 +18,13 @@ constexpr int kBufferFlags = 0x00020000;  // raw buffer resource word 3 on gfx9
 // consecutive rows free of LDS bank conflicts (8- and 16-lane phases).
 __device__ __forceinline__ int swz_a(int r) { return ((r >> 1) & 3) ^ ((r >> 3) & 1); }
 
+// A-side rows of 128 bytes (8 chunks): chunk c of row r is stored at chunk
+// c ^ swz_a2(r). For the operand reads (32 consecutive rows, one logical chunk
+// per half wave) every 8 consecutive rows land on 8 distinct 16-byte bank
+// groups and every 16 on 16 distinct (row parity, chunk) pairs: no bank
+// conflicts for 8- or 16-lane LDS phases.
+__device__ __forceinline__ int swz_a2(int r) { return ((r >> 1) & 7) ^ ((r & 1) << 2); }
+
 // Wait until at most N vector-memory operations of this wave are pending and
 // its LDS operations have drained, then join the workgroup barrier. The empty
 // asm with a memory clobber keeps the compiler from moving LDS accesses
@@ -45,7 +52,21 @@ __device__ __forceinline__ void lds_dma16(__amdgpu_buffer_rsrc_t rsrc, unsigned 
                  : "s"(lds_addr), "v"(voff), "s"(rsrc), "s"(soff)
                  : "memory", "m0");
 }
+// The same with 4 bytes per lane (256 LDS bytes per instruction): sources on 4 bytes.
+__device__ __forceinline__ void lds_dma4(__amdgpu_buffer_rsrc_t rsrc, unsigned lds_addr, int voff, int soff) {
+    asm volatile("s_mov_b32 m0, %0\n\tbuffer_load_dword %1, %2, %3 offen lds"
+                 :
+                 : "s"(lds_addr), "v"(voff), "s"(rsrc), "s"(soff)
+                 : "memory", "m0");
+}
 #pragma clang diagnostic pop
+
+template <int BYTES>
+__device__ __forceinline__ void lds_dma(__amdgpu_buffer_rsrc_t rsrc, unsigned lds_addr, int voff, int soff) {
+    static_assert(BYTES == 16 || BYTES == 4, "bytes per lane of an LDS-DMA load");
+    if constexpr (BYTES == 16) lds_dma16(rsrc, lds_addr, voff, soff);
+    else lds_dma4(rsrc, lds_addr, voff, soff);
+}
 
 // Tile index -> (tile row, tile column). Blocks are dispatched round-robin
 // over the 8 XCDs (block b on XCD b % 8); each XCD gets a contiguous range of

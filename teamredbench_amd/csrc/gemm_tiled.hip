@@ -136,14 +136,6 @@ struct Traits<MB_DT_FLOAT8_E5M2> : Traits<MB_DT_FLOAT8_E4M3FN> {
     }
 };
 
-// A is held two stages at a time: rows of 128 bytes (stage 2p in chunks 0-3,
-// stage 2p + 1 in chunks 4-7), chunk c of row r stored at chunk c ^ swz_a2(r).
-// For the operand reads (32 consecutive rows, one logical chunk per half
-// wave) every 8 consecutive rows land on 8 distinct 16-byte bank groups and
-// every 16 on 16 distinct (row parity, chunk) pairs: no bank conflicts for 8-
-// or 16-lane LDS phases.
-__device__ __forceinline__ int swz_a2(int r) { return ((r >> 1) & 7) ^ ((r & 1) << 2); }
-
 // One 16-byte piece of this lane's A operand: row `row` of the pair slot,
 // 16-byte K chunk `chunk` (0..7: 4 * stage parity + chunk within the stage;
 // 16-bit: chunk 2s + lane/32 of substep s; fp8: chunks 2*(lane/32) and +1

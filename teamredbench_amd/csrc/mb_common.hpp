@@ -125,7 +125,10 @@ struct GemmPlan {
     int config = 0;             // configuration within the family
 };
 
-int gemm_plan(int dtype, int64_t M, int64_t N, int64_t K, const DeviceProps& props,
+// `scratch`: the largest workspace the caller can give to plans that use one
+// only to run faster (a caller that gives none still gets a plan without it).
+// Plans that cannot do without a workspace ask for it whatever `scratch` is.
+int gemm_plan(int dtype, int64_t M, int64_t N, int64_t K, const DeviceProps& props, size_t scratch,
               GemmPlan* plan);
 
 // One launch of the MFMA-only kernel of instruction `kind` (MB_MFMA_*).

@@ -197,6 +197,44 @@ def test_full_precision_ring_on_partial_tiles(lib, dtype, shape):
     assert (np.abs(got_all[rows] - ref) <= bound + 1e-300).all()
 
 
+# (M, N, K) -> tile, split over K when a workspace is given: one row, remainders of every tile, rows off 16
+# bytes (4-byte DMA pieces), a K off the stage, the last split running past K.
+RING_TILES = [
+    ((1, 1024, 1027), None, True), ((33, 1030, 520), None, True), ((5, 4099, 2051), (32, 128), True),
+    ((7, 4096, 2048), (32, 128), True), ((600, 704, 1904), None, True), ((601, 703, 1905), None, True),
+    ((130, 2050, 1111), None, True), ((100, 640, 640), None, True),
+    ((900, 1000, 300), (128, 32), False), ((901, 999, 301), (128, 32), False),
+    ((513, 515, 97), (128, 128), False), ((2048, 2048, 136), (128, 128), False),
+]
+
+
+@pytest.mark.parametrize("dtype", ["float32", "float64"])
+@pytest.mark.parametrize("shape, tile, splits", RING_TILES)
+def test_full_precision_tiles_and_splits(lib, dtype, shape, tile, splits):
+    # Every element within the accumulation bound of an fp64 matmul, with the workspace the plan asks for and
+    # without one (no split then), nothing written past C or the workspace.
+    m, n, k = shape
+    dt, tdt = capi.DTYPES[dtype], getattr(torch, dtype)
+    info = lib.gemm_info(dt, m, n, k)
+    print(f"[gemm-ragged] {dtype} {m}x{n}x{k}: {info['tile_m']}x{info['tile_n']} split {info['split_k']}", flush=True)
+    assert (info["split_k"] > 1) is splits and (tile is None or (info["tile_m"], info["tile_n"]) == tile), info
+    ops = rp.gemm_inputs(m, n, k, dtype, seed=m + k)
+    da, db = ops["a"].cuda(), ops["b"].cuda()
+    a64, b64 = ops["a"].double().numpy(), ops["b"].double().numpy()
+    ref = a64 @ b64
+    bound = elementwise_bound(dtype, k, np.abs(ref), np.abs(a64) @ np.abs(b64))
+    for ws_bytes in (lib.gemm_workspace_size(dt, m, n, k), 0):
+        flat = torch.full((m * n + GUARD,), float("nan"), dtype=tdt, device="cuda")
+        ws = torch.full((ws_bytes + GUARD,), 0x7F, dtype=torch.uint8, device="cuda")
+        lib.gemm(dt, da.data_ptr(), db.data_ptr(), flat.data_ptr(), m, n, k, 1.0, 1.0,
+                 ws.data_ptr() if ws_bytes else None, ws_bytes, torch.cuda.current_stream().cuda_stream)
+        torch.cuda.synchronize()
+        assert torch.isnan(flat[m * n:]).all(), "the GEMM wrote past the end of C"
+        assert (ws[ws_bytes:] == 0x7F).all(), "the GEMM wrote past the end of its workspace"
+        got = flat[: m * n].view(m, n).cpu().double().numpy()
+        assert (np.abs(got - ref) <= bound).all(), f"workspace {ws_bytes}: off by {np.abs(got - ref).max()}"
+
+
 # Shapes whose B passes 2^31 bytes, with the kernel each must run on.
 BEYOND_32_BIT = [
     ("bfloat16", 65536, GENERIC),                     # B 4 GiB
