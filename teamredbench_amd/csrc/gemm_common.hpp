@@ -75,6 +75,15 @@ int gemm_tiled_plan(int dtype, int64_t M, int64_t N, int64_t K, const DeviceProp
                     GemmPlan* plan, const char** why);
 int gemm_tiled_launch(int dtype, const void* A, const void* B, void* C, int64_t M, int64_t N,
                       int64_t K, float alpha, void* workspace, const GemmPlan& plan, hipStream_t stream);
+// One per input type (gemm_tiled_<type>.hip).
+int gemm_tiled_launch_bf16(const GemmPlan& plan, const void* A, const void* B, void* C, int64_t M, int64_t N,
+                           int64_t K, float alpha, void* workspace, hipStream_t stream);
+int gemm_tiled_launch_f16(const GemmPlan& plan, const void* A, const void* B, void* C, int64_t M, int64_t N,
+                           int64_t K, float alpha, void* workspace, hipStream_t stream);
+int gemm_tiled_launch_e4m3(const GemmPlan& plan, const void* A, const void* B, void* C, int64_t M, int64_t N,
+                           int64_t K, float alpha, void* workspace, hipStream_t stream);
+int gemm_tiled_launch_e5m2(const GemmPlan& plan, const void* A, const void* B, void* C, int64_t M, int64_t N,
+                           int64_t K, float alpha, void* workspace, hipStream_t stream);
 int gemm_generic_launch(int dtype, const void* A, const void* B, void* C, int64_t M, int64_t N,
                         int64_t K, float alpha, hipStream_t stream);
 int gemm_highp_plan(int dtype, int64_t M, int64_t N, int64_t K, const DeviceProps& props, size_t scratch,
