@@ -106,16 +106,16 @@ int mb_time_stream(int op, int dtype, void* dst, const void* b, const void* c,
  * FLOAT64      fp64        fp64        fp64        fp64 MFMA
  * scale_a/scale_b are the fp8 per-tensor dequantisation scales (ignored for
  * the other types). Leading dimensions are K, N and N. Any M, N, K >= 1 with
- * 16-byte aligned base pointers; shapes the pipelined kernels do not divide
- * (N % 128, K % 64 bytes) run on bounds-checked kernels.
+ * 16-byte aligned base pointers.
  * FLOAT32 / FLOAT64 follow the reference's high-precision path
  * (mfu_gemm_highp.hip.hpp:39-218) on v_mfma_f32_32x32x2_f32 and
  * v_mfma_f64_16x16x4_f64; FLOAT8_E5M2 is the dtype the reference declares
  * (dtypes.py:24) but does not run natively (mfu_gemm.hip.cpp:9-21).
  * workspace: device scratch of at least mb_gemm_workspace_size() bytes (may
  * be NULL when that size is 0). The kernels leave it in a state the next
- * call can use without clearing. FLOAT32 / FLOAT64 use it to run faster (K
- * split over idle CUs): with less than that size, or NULL, they run without.
+ * call can use without clearing. FLOAT32 / FLOAT64 (K split over idle CUs) and
+ * the other types with rows off 16 bytes (operands repacked) use it only to run
+ * faster: with less than that size, or NULL, they run without.
  */
 int mb_gemm(int dtype, const void* A, const void* B, void* C, int64_t M,
             int64_t N, int64_t K, float scale_a, float scale_b, void* workspace,
@@ -130,8 +130,8 @@ size_t mb_gemm_workspace_size(int dtype, int64_t M, int64_t N, int64_t K);
  * harnesses that forbid hipMalloc). It has no counterpart in the reference.
  *
  * Same arguments, kernels and results as mb_gemm (as mb_gemm without a
- * workspace for FLOAT32 / FLOAT64, which use no scratch here). The split-K /
- * small-M partial sums go to a library-owned device array of
+ * workspace where that is optional). The split-K / small-M partial sums go to
+ * a library-owned device array of
  * MB_NOALLOC_SCRATCH_BYTES per GPU, which each GPU holds until the process
  * ends; the call itself allocates nothing. Shapes whose plan needs more
  * scratch than that return MB_ERR_WORKSPACE before any launch. The first

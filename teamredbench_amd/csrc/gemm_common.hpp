@@ -10,6 +10,7 @@ enum GemmVariant {
     kVariantGeneric = 0,  // any shape, bounds-checked (gemm_generic.hip)
     kVariantTiled = 1,    // N % 256, LDS-DMA pipelined, optional split-K (gemm_tiled.hip)
     kVariantHighp = 2,    // fp32 / fp64 inputs, any shape (gemm_highp.hip)
+    kVariantPacked = 4,   // the tiled kernels on operands repacked to 16-byte rows (gemm_pack.hip)
     kVariantGemv = 3,     // bf16 / fp16 with M <= 4: streaming FMA kernel (gemm_gemv.hip)
 };
 
@@ -86,6 +87,12 @@ int gemm_tiled_launch_e5m2(const GemmPlan& plan, const void* A, const void* B, v
                            int64_t K, float alpha, void* workspace, hipStream_t stream);
 int gemm_generic_launch(int dtype, const void* A, const void* B, void* C, int64_t M, int64_t N,
                         int64_t K, float alpha, hipStream_t stream);
+// The tiled kernels on repacked operands, for rows off 16 bytes: MB_ERR_SHAPE
+// when they cannot take the shape, would not pay, or need more than `scratch`.
+int gemm_packed_plan(int dtype, int64_t M, int64_t N, int64_t K, const DeviceProps& props, size_t scratch,
+                     GemmPlan* plan);
+int gemm_packed_launch(int dtype, const void* A, const void* B, void* C, int64_t M, int64_t N, int64_t K,
+                       float alpha, void* workspace, const GemmPlan& plan, hipStream_t stream);
 int gemm_highp_plan(int dtype, int64_t M, int64_t N, int64_t K, const DeviceProps& props, size_t scratch,
                     GemmPlan* plan);
 int gemm_gemv_plan(int dtype, int64_t M, int64_t N, int64_t K, const DeviceProps& props, GemmPlan* plan);

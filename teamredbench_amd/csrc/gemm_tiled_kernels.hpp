@@ -273,6 +273,8 @@ __device__ __forceinline__ u32x2 pack4(float a, float b, float c, float d) {
     }
 }
 
+typedef u32x4 u32x4_2 __attribute__((aligned(2)));   // 16 bytes at any even address
+
 // Second half of the epilogue: a wave's (WTM x ROW_BYTES / 2) tile, staged in
 // LDS as 16-bit values (chunk c of row r at chunk c ^ (r % chunks)), read back
 // row by row and stored so that 16 (8, 4) lanes write one 256-byte (128-,
@@ -283,8 +285,10 @@ __device__ __forceinline__ u32x2 pack4(float a, float b, float c, float d) {
 // L2 lets the burst drain faster (measured +0.6% at 8192^3, +1.8% at 4096^3,
 // +2.6% at fp8 8192 x 1024 x 8192). Rows at or past M (a partial last tile)
 // and 8-column chunks at or past N (a partial last tile of a ragged N, which
-// is a multiple of 8) are not stored.
-template <int WTM, int ROW_BYTES>
+// is a multiple of 8) are not stored. ANY_N (any N, so C's rows start on any
+// even byte): the columns of the chunk that straddles N go out one by one, and
+// the stores are ordinary ones, since neighbouring tiles share cache lines.
+template <int WTM, int ROW_BYTES, bool ANY_N>
 __device__ __forceinline__ void store_staged_tile(const unsigned char* stage, unsigned char* C, int M, int N,
                                                   int row_base, int64_t col_base, int lane) {
     constexpr int ROW_CHUNKS = ROW_BYTES / 16;
@@ -296,6 +300,7 @@ __device__ __forceinline__ void store_staged_tile(const unsigned char* stage, un
     const int c = lane % ROW_CHUNKS;
     const int r0 = lane / ROW_CHUNKS;
     const bool col_in = col_base + 8 * c < N;
+    const int left = N - (int)(col_base + 8 * c);   // columns of C from the chunk on
     int grow = row_base + r0;
     unsigned char* cptr = C + (int64_t)grow * ldc + col_base * 2 + c * 16;
 #pragma unroll
@@ -308,18 +313,28 @@ __device__ __forceinline__ void store_staged_tile(const unsigned char* stage, un
         }
 #pragma unroll
         for (int p = 0; p < BATCH; ++p) {
-            if (grow < M && col_in) __builtin_nontemporal_store(rows[p], reinterpret_cast<u32x4*>(cptr));
+            if constexpr (ANY_N) {
+                if (grow < M && left >= 8) {
+                    *reinterpret_cast<u32x4_2*>(cptr) = rows[p];
+                } else if (grow < M && left > 0) {
+#pragma unroll
+                    for (int e = 0; e < 7; ++e)
+                        if (e < left) reinterpret_cast<uint16_t*>(cptr)[e] = (uint16_t)(rows[p][e >> 1] >> 16 * (e & 1));
+                }
+            } else {
+                if (grow < M && col_in) __builtin_nontemporal_store(rows[p], reinterpret_cast<u32x4*>(cptr));
+            }
             grow += ROWS_PER_STORE;
             cptr += ROWS_PER_STORE * ldc;
         }
     }
 }
 
-template <int DT, int BM, int BN, int WGM, int WGN, int NA, int NB, bool SCALED, bool RAGGED_K = false>
+template <int DT, int BM, int BN, int WGM, int WGN, int NA, int NB, bool SCALED, bool RAGGED_K, bool ANY_N>
 __global__ void __launch_bounds__(64 * WGM * WGN)
 gemm_tiled_kernel(const unsigned char* __restrict__ A, const unsigned char* __restrict__ B,
-                  unsigned char* __restrict__ C, int M, int N, int K, float alpha, int tiles_m,
-                  int tiles_n, int group_m, int splits, int k_len, float* __restrict__ ws) {
+                  unsigned char* __restrict__ C, int M, int N, int K, int lda, int ldb, int ldp, float alpha,
+                  int tiles_m, int tiles_n, int group_m, int splits, int k_len, float* __restrict__ ws) {
     typedef Traits<DT> Tr;
     typedef typename Tr::Frag Frag;
     constexpr int W = WGM * WGN;
@@ -366,8 +381,7 @@ gemm_tiled_kernel(const unsigned char* __restrict__ A, const unsigned char* __re
     const int tile = splits > 1 ? (int)blockIdx.x / splits : (int)blockIdx.x;
     int tm, tn;
     tile_coords(tile, tiles_m * tiles_n, tiles_m, tiles_n, group_m, &tm, &tn);
-    const int lda = K * E;   // bytes per A row
-    const int ldb = N * E;   // bytes per B row
+    // lda, ldb: bytes per A and B row; ldp: columns per row of a partial plane.
     const int k0 = split * k_len;  // first K element of this block
 
     // Buffer resources over this block's A row panel and B column panel. The A
@@ -646,24 +660,24 @@ gemm_tiled_kernel(const unsigned char* __restrict__ A, const unsigned char* __re
                 [&]<int... I>(std::integer_sequence<int, I...>) {
                     (stage_row(std::integral_constant<int, grp * (GROUP / 32) + I>{}), ...);
                 }(std::make_integer_sequence<int, GROUP / 32>{});
-                store_staged_tile<GROUP, ROW_BYTES>(stage + GROUP * grp * ROW_BYTES, C, M, N,
+                store_staged_tile<GROUP, ROW_BYTES, ANY_N>(stage + GROUP * grp * ROW_BYTES, C, M, N,
                                                     tm * BM + wm * WTM + GROUP * grp, (int64_t)tn * BN + wn * WTN, lane);
             }(), ...);
         }(std::make_integer_sequence<int, WTM / GROUP>{});
     } else if constexpr (BM <= 128) {
-        float* part = ws + (int64_t)split * M * N;
+        float* part = ws + (int64_t)split * M * ldp;
 #pragma unroll
         for (int i = 0; i < FM; ++i) {
             if (row0 + 32 * i >= M) continue;
-            float* prow = part + (int64_t)(row0 + 32 * i) * N;
+            float* prow = part + (int64_t)(row0 + 32 * i) * ldp;
 #pragma unroll
             for (int j = 0; j < FN; ++j) {
 #pragma unroll
                 for (int g = 0; g < 4; ++g) {
                     const f32x16& v = acc[i][j];
                     const f32x4 q = {v[4 * g], v[4 * g + 1], v[4 * g + 2], v[4 * g + 3]};
-                    // N is a multiple of 8: the 4 columns are all in C or all past it
-                    if (col0 + 32 * j + 8 * g < N) *reinterpret_cast<f32x4*>(prow + col0 + 32 * j + 8 * g) = q;
+                    // ldp is a multiple of 8: the 4 columns are all in the plane or all past it
+                    if (col0 + 32 * j + 8 * g < ldp) *reinterpret_cast<f32x4*>(prow + col0 + 32 * j + 8 * g) = q;
                 }
             }
         }
@@ -711,11 +725,11 @@ __device__ __forceinline__ f32x4 mfma16_fp8(const i32x8& a, const i32x8& b, f32x
     return __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(a, b, c, fmt, fmt, 0, 0, 0, 0);
 }
 
-template <int DT, int BM, int BN, int WGM, int WGN, int NA, int NB, bool SCALED, bool RAGGED_K = false>
+template <int DT, int BM, int BN, int WGM, int WGN, int NA, int NB, bool SCALED, bool RAGGED_K, bool ANY_N>
 __global__ void __launch_bounds__(64 * WGM * WGN)
 gemm_fp8_mi16_kernel(const unsigned char* __restrict__ A, const unsigned char* __restrict__ B,
-                     unsigned char* __restrict__ C, int M, int N, int K, float alpha, int tiles_m, int tiles_n,
-                     int group_m, int splits, int k_len, float* __restrict__ ws) {
+                     unsigned char* __restrict__ C, int M, int N, int K, int lda, int ldb, int ldp, float alpha,
+                     int tiles_m, int tiles_n, int group_m, int splits, int k_len, float* __restrict__ ws) {
     constexpr int W = WGM * WGN;
     constexpr int WTM = BM / WGM, WTN = BN / WGN;
     constexpr int FM = WTM / 16, FN = WTN / 16;
@@ -756,7 +770,6 @@ gemm_fp8_mi16_kernel(const unsigned char* __restrict__ A, const unsigned char* _
     const int tile = splits > 1 ? (int)blockIdx.x / splits : (int)blockIdx.x;
     int tm, tn;
     tile_coords(tile, tiles_m * tiles_n, tiles_m, tiles_n, group_m, &tm, &tn);
-    const int lda = K, ldb = N;
     const int k0 = split * k_len;
 
     const int a_rows = min(BM, M - tm * BM);
@@ -1000,21 +1013,21 @@ gemm_fp8_mi16_kernel(const unsigned char* __restrict__ A, const unsigned char* _
                         *reinterpret_cast<u32x2*>(stage + r * ROW_BYTES + chunk * 16 + 8 * (g & 1)) = packed;
                     }
                 }
-                store_staged_tile<GROUP, ROW_BYTES>(stage + GROUP * p * ROW_BYTES, C, M, N, tm * BM + wm * WTM + GROUP * p,
+                store_staged_tile<GROUP, ROW_BYTES, ANY_N>(stage + GROUP * p * ROW_BYTES, C, M, N, tm * BM + wm * WTM + GROUP * p,
                                                     (int64_t)tn * BN + wn * WTN, lane);
             }(), ...);
         }(std::make_integer_sequence<int, WTM / GROUP>{});
     } else if constexpr (BM <= 128) {
-        float* part = ws + (int64_t)split * M * N;
+        float* part = ws + (int64_t)split * M * ldp;
         const int row0 = tm * BM + wm * WTM + l16;
         const int64_t col0 = (int64_t)tn * BN + wn * WTN + 4 * g;
 #pragma unroll
         for (int i = 0; i < FM; ++i) {
             if (row0 + 16 * i >= M) continue;
-            float* prow = part + (int64_t)(row0 + 16 * i) * N;
+            float* prow = part + (int64_t)(row0 + 16 * i) * ldp;
 #pragma unroll
             for (int j = 0; j < FN; ++j)
-                if (col0 + 16 * j < N) *reinterpret_cast<f32x4*>(prow + col0 + 16 * j) = acc[i][j];
+                if (col0 + 16 * j < ldp) *reinterpret_cast<f32x4*>(prow + col0 + 16 * j) = acc[i][j];
         }
     }
 }
@@ -1024,10 +1037,11 @@ gemm_fp8_mi16_kernel(const unsigned char* __restrict__ A, const unsigned char* _
 // L splits' loads in flight at once, L the split count rounded up to a power
 // of two (at most 32): the planes were just written by the GEMM kernel, so
 // the pass is latency-bound. The adds keep split order.
-template <int DT, int L>
+// ANY_N: planes have rows of ldp columns and C rows of N, any N.
+template <int DT, int L, bool ANY_N>
 __global__ void __launch_bounds__(256)
 gemm_splitk_reduce_kernel(const float* __restrict__ ws, unsigned char* __restrict__ C, int64_t quads,
-                          int64_t plane, int splits, float alpha) {
+                          int64_t plane, int splits, float alpha, int N, int ldp) {
     constexpr int kLoads = L;
     const int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (q >= quads) return;
@@ -1042,7 +1056,21 @@ gemm_splitk_reduce_kernel(const float* __restrict__ ws, unsigned char* __restric
         for (int u = 0; u < kLoads; ++u)
             if (s0 + u < splits) sum += v[u];
     }
-    *reinterpret_cast<u32x2*>(C + 8 * q) = pack4<DT>(sum[0] * alpha, sum[1] * alpha, sum[2] * alpha, sum[3] * alpha);
+    const u32x2 c4 = pack4<DT>(sum[0] * alpha, sum[1] * alpha, sum[2] * alpha, sum[3] * alpha);
+    if constexpr (ANY_N) {
+        typedef u32x2 u32x2_2 __attribute__((aligned(2)));
+        const int row = (int)(q / (ldp >> 2)), col = 4 * (int)(q - (int64_t)row * (ldp >> 2));
+        uint16_t* p = reinterpret_cast<uint16_t*>(C) + (int64_t)row * N + col;
+        if (col + 4 <= N) {
+            *reinterpret_cast<u32x2_2*>(p) = c4;
+        } else {
+#pragma unroll
+            for (int e = 0; e < 3; ++e)
+                if (col + e < N) p[e] = (uint16_t)(c4[e >> 1] >> 16 * (e & 1));
+        }
+    } else {
+        *reinterpret_cast<u32x2*>(C + 8 * q) = c4;
+    }
 }
 
 struct TiledConfig {
@@ -1070,8 +1098,8 @@ int launch_cfg(const void* A, const void* B, void* C, int64_t M, int64_t N, int6
     auto* cp = static_cast<unsigned char*>(C);
     // Only fp8 carries a scale; the split-K partials are scaled by the reduction.
     // fp8 runs the 16x16x128 kernel when the plan says so (frag_m 16).
-    typedef void (*Kernel)(const unsigned char*, const unsigned char*, unsigned char*, int, int, int, float, int,
-                           int, int, int, int, float*);
+    typedef void (*Kernel)(const unsigned char*, const unsigned char*, unsigned char*, int, int, int, int, int, int,
+                           float, int, int, int, int, int, float*);
     const bool scaled = is_fp8(DT) && alpha != 1.0f && splits == 1;
     // K not a multiple of splits x stage: every split runs k_len (whole
     // stages), and the instantiations with RAGGED_K zero the A pieces past K.
@@ -1079,29 +1107,40 @@ int launch_cfg(const void* A, const void* B, void* C, int64_t M, int64_t N, int6
     const int64_t stages = (K + stage_k - 1) / stage_k;
     const int64_t k_len = (stages + splits - 1) / splits * stage_k;   // the plan's split_k_len
     const bool ragged_k = k_len * splits != K;
-    auto pick = [&](auto rk) -> Kernel {
-        constexpr bool RK = decltype(rk)::value;
+    const bool any_n = plan.packed;   // repacked operands: any N and K, C's rows on any even byte
+    auto pick = [&](auto rk, auto an) -> Kernel {
+        constexpr bool RK = decltype(rk)::value, AN = decltype(an)::value;
         if constexpr (is_fp8(DT)) {
             if constexpr (c.bn >= 128) {   // the 16x16x128 kernel's B swizzles cover rows of 128 bytes or more
                 if (plan.frag_m == 16)
-                    return scaled ? gemm_fp8_mi16_kernel<DT, c.bm, c.bn, c.wgm, c.wgn, c.na, c.nb, true, RK>
-                                  : gemm_fp8_mi16_kernel<DT, c.bm, c.bn, c.wgm, c.wgn, c.na, c.nb, false, RK>;
+                    return scaled || AN ? gemm_fp8_mi16_kernel<DT, c.bm, c.bn, c.wgm, c.wgn, c.na, c.nb, true, RK, AN>
+                                        : gemm_fp8_mi16_kernel<DT, c.bm, c.bn, c.wgm, c.wgn, c.na, c.nb, AN, RK, AN>;
             }
-            if (scaled) return gemm_tiled_kernel<DT, c.bm, c.bn, c.wgm, c.wgn, c.na, c.nb, true, RK>;
+            if (scaled || AN) return gemm_tiled_kernel<DT, c.bm, c.bn, c.wgm, c.wgn, c.na, c.nb, true, RK, AN>;
         }
-        return gemm_tiled_kernel<DT, c.bm, c.bn, c.wgm, c.wgn, c.na, c.nb, false, RK>;
+        return gemm_tiled_kernel<DT, c.bm, c.bn, c.wgm, c.wgn, c.na, c.nb, is_fp8(DT) && AN, RK, AN>;
     };
-    const Kernel kernel = ragged_k ? pick(std::true_type{}) : pick(std::false_type{});
-    hipLaunchKernelGGL(kernel, grid, block, 0, stream, a, b, cp, (int)M, (int)N, (int)K, scaled ? alpha : 1.0f,
-                       tiles_m, tiles_n, c.group_m, splits, (int)k_len, ws);
+    const Kernel kernel = any_n ? pick(std::true_type{}, std::true_type{})
+                        : ragged_k ? pick(std::true_type{}, std::false_type{})
+                                   : pick(std::false_type{}, std::false_type{});
+    constexpr int E = Traits<DT>::kElem;
+    const int lda = any_n ? (int)plan.lda : (int)K * E, ldb = any_n ? (int)plan.ldb : (int)N * E;
+    const int ldp = (int)((N + 7) / 8 * 8);
+    hipLaunchKernelGGL(kernel, grid, block, 0, stream, a, b, cp, (int)M, (int)N, (int)K, lda, ldb, ldp,
+                       scaled ? alpha : 1.0f, tiles_m, tiles_n, c.group_m, splits, (int)k_len, ws);
     MB_HIP_TRY(hipGetLastError());
     if (splits > 1) {
-        const int64_t quads = M * N / 4;
-        auto reduce = splits <= 4 ? gemm_splitk_reduce_kernel<DT, 4>
-                    : splits <= 8 ? gemm_splitk_reduce_kernel<DT, 8>
-                    : splits <= 16 ? gemm_splitk_reduce_kernel<DT, 16> : gemm_splitk_reduce_kernel<DT, 32>;
+        const int64_t quads = M * ldp / 4;
+        auto reduce_for = [&](auto an) {
+            constexpr bool AN = decltype(an)::value;
+            return splits <= 4 ? gemm_splitk_reduce_kernel<DT, 4, AN>
+                 : splits <= 8 ? gemm_splitk_reduce_kernel<DT, 8, AN>
+                 : splits <= 16 ? gemm_splitk_reduce_kernel<DT, 16, AN> : gemm_splitk_reduce_kernel<DT, 32, AN>;
+        };
+        auto reduce = any_n ? reduce_for(std::true_type{}) : reduce_for(std::false_type{});
         hipLaunchKernelGGL(reduce, dim3((unsigned)((quads + 255) / 256)), dim3(256), 0, stream,
-                           static_cast<const float*>(ws), static_cast<unsigned char*>(C), quads, M * N, splits, alpha);
+                           static_cast<const float*>(ws), static_cast<unsigned char*>(C), quads, M * ldp, splits, alpha,
+                           (int)N, ldp);
         MB_HIP_TRY(hipGetLastError());
     }
     return MB_OK;

@@ -121,6 +121,12 @@ struct GemmPlan {
     int tile_group_m = 0;
     size_t workspace = 0;
     const char* fallback = "";  // why a faster kernel family could not take the shape ("" if none)
+    // Operands repacked into the workspace first (rows off 16 bytes): bytes per
+    // row of A and B as the GEMM reads them, and where the repacked operands
+    // (0: none, read in place) and the partial planes start in the workspace.
+    bool packed = false, pack_a = false, pack_b = false;
+    int64_t lda = 0, ldb = 0;
+    size_t a_offset = 0, b_offset = 0, partials_offset = 0;
     int variant = 0;            // kernel family selector, private to gemm*.hip
     int config = 0;             // configuration within the family
 };

@@ -158,6 +158,30 @@ def test_shapes_off_the_pipelined_kernels(lib, dtype, shape):
     assert info["implementation"] == GENERIC and info["fallback"] != "", info
 
 
+# Rows off 16 bytes: N off, K off, both, by one element either side of a multiple; one row; a K shorter than a
+# piece; tile remainders; unsplit and split plans; a partial last piece in the last row of A and of B.
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("shape", [(300, 513, 512), (300, 512, 511), (257, 255, 1025), (64, 1030, 4099),
+                                   (1, 1025, 2049), (40, 2047, 3), (520, 130, 77), (1024, 1279, 1281)])
+def test_rows_off_16_bytes(lib, dtype, shape):
+    # The same operands with the workspace the plan asks for (repacked) and without one (bounds-checked kernel).
+    m, n, k = shape
+    dt = capi.DTYPES[dtype]
+    run_checked(lib, dtype, *shape, seed=m)
+    ops = rp.gemm_inputs(m, n, k, dtype, seed=m)
+    da, db = ops["a"].cuda(), ops["b"].cuda()
+    flat = torch.full((m * n + GUARD,), float("nan"), dtype=rp.gemm_output_dtype(dtype), device="cuda")
+    lib.gemm(dt, da.data_ptr(), db.data_ptr(), flat.data_ptr(), m, n, k, ops["scale_a"], ops["scale_b"], None, 0,
+             torch.cuda.current_stream().cuda_stream)
+    torch.cuda.synchronize()
+    assert torch.isnan(flat[m * n:].float()).all(), "the GEMM wrote past the end of C"
+    got = flat[: m * n].view(m, n).cpu().double().numpy()
+    a64, b64 = ops["a"].double().numpy(), ops["b"].double().numpy()
+    scale = float(ops["scale_a"]) * float(ops["scale_b"])
+    ref = scale * (a64 @ b64)
+    assert (np.abs(got - ref) <= elementwise_bound(dtype, k, np.abs(ref), scale * (np.abs(a64) @ np.abs(b64)))).all()
+
+
 @pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("shape", [(1, 1, 1), (7, 9, 11), (256, 256, 512), (129, 257, 96), (5, 3000, 8),
                                    (300, 1008, 512), (1024, 1024, 1024)])
