@@ -748,8 +748,8 @@ HighpChoice highp_choose(bool f64, int64_t M, int64_t N, int64_t K, int cus, siz
     }
     // 128 x 128 tiles where they fill whole rounds exactly, and for K of a few
     // stages, where the tile hardly matters. fp64 with one block per CU takes
-    // 128-byte rows of A (2048^3 251 against 261 us; with more blocks their
-    // 128 KiB of ring leave one block per CU and run 4-9% slower).
+    // 128-byte rows of A (2048^3 249 against 254 us; with more blocks their
+    // 128 KiB of ring leave one block per CU and run 8-9% slower).
     if ((M % 128 == 0 && N % 128 == 0 && tiles(2) % cus == 0) || (K < 128 && M >= 512)) {
         ch.config = f64 && tiles(2) <= cus && K >= 128 ? 3 : 2;
         return ch;
@@ -791,6 +791,8 @@ HighpChoice highp_choose(bool f64, int64_t M, int64_t N, int64_t K, int cus, siz
             if (best < 0.0 || t < best) best = t, ch.config = c, ch.splits = sp;
         }
     }
+    // fp64 alone on a CU: 128-byte rows of A (above).
+    if (f64 && ch.config == 2 && tiles(2) * ch.splits <= cus && k_len(3, ch.splits) * (ch.splits - 1) < K) ch.config = 3;
     // One unsplit round of at least six 128-row panels runs 128 x 32 tiles:
     // 128-row tiles without a workspace are what a plan of 1000^3 has always
     // reported (26.7 us fp32 and 41.9 fp64, against 65 and 123 on 128 x 128;
