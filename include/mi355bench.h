@@ -114,7 +114,7 @@ int mb_time_stream(int op, int dtype, void* dst, const void* b, const void* c,
  * workspace: device scratch of at least mb_gemm_workspace_size() bytes (may
  * be NULL when that size is 0). The kernels leave it in a state the next
  * call can use without clearing. FLOAT32 / FLOAT64 (K split over idle CUs) and
- * the other types with rows off 16 bytes (operands repacked) use it only to run
+ * the other types with rows off 16 bytes (operands repacked, or K split) use it only to run
  * faster: with less than that size, or NULL, they run without.
  */
 int mb_gemm(int dtype, const void* A, const void* B, void* C, int64_t M,

@@ -24,7 +24,10 @@ int gemm_plan(int dtype, int64_t M, int64_t N, int64_t K, const DeviceProps& pro
         return MB_OK;
     const char* why = "forced by the gemm_force_generic override";
     if (!generic_only && gemm_tiled_plan(dtype, M, N, K, props, plan, &why) == MB_OK) return MB_OK;
-    const int rc = !generic_only && gemm_packed_plan(dtype, M, N, K, props, scratch, plan) == MB_OK
+    const int64_t grain = is_fp8(dtype) ? 16 : 8;
+    const bool off16 = N % grain != 0 || K % grain != 0;
+    const int rc = !generic_only && off16 && (gemm_strip_plan(dtype, M, N, K, props, scratch, plan) == MB_OK ||
+                                              gemm_packed_plan(dtype, M, N, K, props, scratch, plan) == MB_OK)
                        ? MB_OK : gemm_generic_plan(dtype, M, N, K, plan);
     plan->fallback = why;
     return rc;
@@ -41,6 +44,8 @@ int gemm_launch(int dtype, const void* A, const void* B, void* C, int64_t M, int
             return gemm_tiled_launch(dtype, A, B, C, M, N, K, alpha, workspace, plan, stream);
         case kVariantPacked:
             return gemm_packed_launch(dtype, A, B, C, M, N, K, alpha, workspace, plan, stream);
+        case kVariantStrip:
+            return gemm_strip_launch(dtype, A, B, C, M, N, K, alpha, workspace, plan, stream);
         case kVariantHighp:
             return gemm_highp_launch(dtype, A, B, C, M, N, K, plan, workspace, stream);
         case kVariantGemv:

@@ -12,6 +12,7 @@ enum GemmVariant {
     kVariantHighp = 2,    // fp32 / fp64 inputs, any shape (gemm_highp.hip)
     kVariantPacked = 4,   // the tiled kernels on operands repacked to 16-byte rows (gemm_pack.hip)
     kVariantGemv = 3,     // bf16 / fp16 with M <= 4: streaming FMA kernel (gemm_gemv.hip)
+    kVariantStrip = 5,    // few rows, rows off 16 bytes: B through registers to the MFMAs (gemm_strip.hip)
 };
 
 constexpr bool is_fp8(int dtype) { return dtype == MB_DT_FLOAT8_E4M3FN || dtype == MB_DT_FLOAT8_E5M2; }
@@ -95,6 +96,13 @@ int gemm_packed_launch(int dtype, const void* A, const void* B, void* C, int64_t
                        float alpha, void* workspace, const GemmPlan& plan, hipStream_t stream);
 int gemm_highp_plan(int dtype, int64_t M, int64_t N, int64_t K, const DeviceProps& props, size_t scratch,
                     GemmPlan* plan);
+// Few rows of A, K or N off 16 bytes; K splits only as far as `scratch` holds their partials.
+int gemm_strip_plan(int dtype, int64_t M, int64_t N, int64_t K, const DeviceProps& props, size_t scratch,
+                    GemmPlan* plan);
+int gemm_strip_launch(int dtype, const void* A, const void* B, void* C, int64_t M, int64_t N, int64_t K,
+                      float alpha, void* workspace, const GemmPlan& plan, hipStream_t stream);
+// C[i] = round(alpha * the sum over `splits` fp32 planes of mn elements) in the output type of `dtype`.
+int gemm_sum_planes(int dtype, const float* ws, void* C, int64_t mn, int splits, float alpha, hipStream_t stream);
 int gemm_gemv_plan(int dtype, int64_t M, int64_t N, int64_t K, const DeviceProps& props, GemmPlan* plan);
 int gemm_gemv_launch(int dtype, const void* A, const void* B, void* C, int64_t M, int64_t N, int64_t K,
                      void* workspace, const GemmPlan& plan, hipStream_t stream);

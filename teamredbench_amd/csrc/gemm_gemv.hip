@@ -41,8 +41,8 @@ __device__ __forceinline__ float elem(unsigned word, int hi) {
 
 template <int DT>
 __device__ __forceinline__ uint16_t round16(float v) {
-    if constexpr (DT == MB_DT_BFLOAT16) return __builtin_bit_cast(uint16_t, (__bf16)v);
-    else return __builtin_bit_cast(uint16_t, (_Float16)v);
+    if constexpr (DT == MB_DT_FLOAT16) return __builtin_bit_cast(uint16_t, (_Float16)v);
+    else return __builtin_bit_cast(uint16_t, (__bf16)v);
 }
 
 template <int DT, int MR>
@@ -117,7 +117,7 @@ gemm_gemv_kernel(const uint16_t* __restrict__ A, const uint16_t* __restrict__ B,
     }
 }
 
-// C[i] = round(sum_s ws[s][i]) over `splits` partial planes of mn elements.
+// C[i] = round(alpha * sum_s ws[s][i]) over `splits` partial planes of mn elements.
 // A block of W waves takes 64 consecutive elements; its wave w adds planes
 // w, w + W, ... with L loads in flight at once, so W * L splits cost one trip
 // to memory (the planes were just written by the previous kernel: the pass is
@@ -131,7 +131,7 @@ constexpr int kGvReduceCols = 64;
 
 template <int DT, int W, int L>
 __global__ void __launch_bounds__(kGvReduceCols * W)
-gemm_gemv_reduce_kernel(const float* __restrict__ ws, uint16_t* __restrict__ C, int64_t mn, int splits) {
+gemm_gemv_reduce_kernel(const float* __restrict__ ws, uint16_t* __restrict__ C, int64_t mn, int splits, float alpha) {
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int64_t i = (int64_t)blockIdx.x * kGvReduceCols + lane;
     float s = 0.f;
@@ -152,12 +152,12 @@ gemm_gemv_reduce_kernel(const float* __restrict__ ws, uint16_t* __restrict__ C, 
     float t = red[0][lane];
 #pragma unroll
     for (int w = 1; w < W; ++w) t += red[w][lane];
-    C[i] = round16<DT>(t);
+    C[i] = round16<DT>(t * alpha);
 }
 
 template <int DT>
-int launch_reduce(const float* ws, uint16_t* C, int64_t mn, int splits, hipStream_t stream) {
-    typedef void (*Reduce)(const float*, uint16_t*, int64_t, int);
+int launch_reduce(const float* ws, uint16_t* C, int64_t mn, int splits, float alpha, hipStream_t stream) {
+    typedef void (*Reduce)(const float*, uint16_t*, int64_t, int, float);
     Reduce reduce = gemm_gemv_reduce_kernel<DT, 16, 32>;
     int waves = 16;
     if (splits <= 4) reduce = gemm_gemv_reduce_kernel<DT, 4, 1>, waves = 4;
@@ -168,7 +168,7 @@ int launch_reduce(const float* ws, uint16_t* C, int64_t mn, int splits, hipStrea
     else if (splits <= 128) reduce = gemm_gemv_reduce_kernel<DT, 16, 8>;
     else if (splits <= 256) reduce = gemm_gemv_reduce_kernel<DT, 16, 16>;
     hipLaunchKernelGGL(reduce, dim3((unsigned)((mn + kGvReduceCols - 1) / kGvReduceCols)),
-                       dim3(kGvReduceCols * waves), 0, stream, ws, C, mn, splits);
+                       dim3(kGvReduceCols * waves), 0, stream, ws, C, mn, splits, alpha);
     MB_HIP_TRY(hipGetLastError());
     return MB_OK;
 }
@@ -184,7 +184,7 @@ int launch_m(const void* A, const void* B, void* C, int64_t M, int64_t N, int64_
                        static_cast<const uint16_t*>(A), static_cast<const uint16_t*>(B), static_cast<uint16_t*>(C),
                        (int)N, (int)K, k_len, ws);
     MB_HIP_TRY(hipGetLastError());
-    if (splits > 1) return launch_reduce<DT>(ws, static_cast<uint16_t*>(C), M * N, splits, stream);
+    if (splits > 1) return launch_reduce<DT>(ws, static_cast<uint16_t*>(C), M * N, splits, 1.0f, stream);
     return MB_OK;
 }
 
@@ -200,6 +200,12 @@ int launch_dt(const void* A, const void* B, void* C, int64_t M, int64_t N, int64
 }
 
 }  // namespace
+
+int gemm_sum_planes(int dtype, const float* ws, void* C, int64_t mn, int splits, float alpha, hipStream_t stream) {
+    return dtype == MB_DT_FLOAT16
+               ? launch_reduce<MB_DT_FLOAT16>(ws, static_cast<uint16_t*>(C), mn, splits, alpha, stream)
+               : launch_reduce<MB_DT_BFLOAT16>(ws, static_cast<uint16_t*>(C), mn, splits, alpha, stream);
+}
 
 // Takes bf16/fp16 with 1 <= M <= 4, N % 8 == 0 and K % 8 == 0 (16-byte
 // loads of B's rows and of A's 8-row chunks); other cases return

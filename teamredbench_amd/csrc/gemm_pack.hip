@@ -4,7 +4,7 @@
 // copies (their DMA loads need 16-byte sources; gemm_tiled_kernels.hpp, ANY_N).
 //
 // The copy is bound by HBM: it reads and writes each repacked operand once, a
-// small part of a product with many rows.
+// small part of a product with many rows (up to 64 go to gemm_strip.hip).
 #include "gemm_common.hpp"
 
 namespace mb {

@@ -182,6 +182,36 @@ def test_rows_off_16_bytes(lib, dtype, shape):
     assert (np.abs(got - ref) <= elementwise_bound(dtype, k, np.abs(ref), scale * (np.abs(a64) @ np.abs(b64)))).all()
 
 
+# Few rows with N or K off 16 bytes: every count of 16-row fragments and its edges, the narrowest N a lane's
+# columns fit, one column past a block, K of one partial step, whole steps only, a partial one after them.
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("splits", [None, 3])
+@pytest.mark.parametrize("shape", [(1, 17, 5), (16, 9, 33), (17, 129, 64), (32, 255, 161), (33, 257, 640),
+                                   (48, 1003, 97), (49, 130, 2049), (64, 2047, 1000), (3, 4096, 1031)])
+def test_few_rows_off_16_bytes(lib, tune, dtype, splits, shape):
+    m, n, k = shape
+    dt = capi.DTYPES[dtype]
+    tune(gemm_splits=splits)
+    run_checked(lib, dtype, *shape, seed=m + n)
+    ops = rp.gemm_inputs(m, n, k, dtype, seed=m + n)
+    da, db = ops["a"].cuda(), ops["b"].cuda()
+    a64, b64 = ops["a"].double().numpy(), ops["b"].double().numpy()
+    scale = float(ops["scale_a"]) * float(ops["scale_b"])
+    ref = scale * (a64 @ b64)
+    bound = elementwise_bound(dtype, k, np.abs(ref), scale * (np.abs(a64) @ np.abs(b64)))
+    need = lib.gemm_workspace_size(dt, m, n, k)
+    for ws_bytes in (need, need // 2, 0):   # all splits, fewer, none
+        flat = torch.full((m * n + GUARD,), float("nan"), dtype=rp.gemm_output_dtype(dtype), device="cuda")
+        ws = torch.full((ws_bytes + GUARD,), 0x7F, dtype=torch.uint8, device="cuda")
+        lib.gemm(dt, da.data_ptr(), db.data_ptr(), flat.data_ptr(), m, n, k, ops["scale_a"], ops["scale_b"],
+                 ws.data_ptr() if ws_bytes else None, ws_bytes, torch.cuda.current_stream().cuda_stream)
+        torch.cuda.synchronize()
+        assert torch.isnan(flat[m * n:].float()).all(), "the GEMM wrote past the end of C"
+        assert (ws[ws_bytes:] == 0x7F).all(), "the GEMM wrote past the end of its workspace"
+        got = flat[: m * n].view(m, n).cpu().double().numpy()
+        assert (np.abs(got - ref) <= bound).all(), f"workspace {ws_bytes}: off by {np.abs(got - ref).max()}"
+
+
 @pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("shape", [(1, 1, 1), (7, 9, 11), (256, 256, 512), (129, 257, 96), (5, 3000, 8),
                                    (300, 1008, 512), (1024, 1024, 1024)])
