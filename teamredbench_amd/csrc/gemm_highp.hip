@@ -283,10 +283,8 @@ gemm_f32_dma_kernel(const float* __restrict__ A, const float* __restrict__ B, fl
     const int tid = threadIdx.x, lane = tid & 63, half = lane >> 5;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wm = wave / WGN, wn = wave % WGN;
-    const int split = splits > 1 ? (int)blockIdx.x % splits : 0;   // the splits of a tile are adjacent
-    const int tile = splits > 1 ? (int)blockIdx.x / splits : (int)blockIdx.x;
-    int tm, tn;
-    tile_coords(tile, tiles_m * tiles_n, tiles_m, tiles_n, kHpGroupM, &tm, &tn);
+    int tm, tn, split;
+    block_coords((int)blockIdx.x, tiles_m, tiles_n, splits, kHpGroupM, &tm, &tn, &split);
     const int lda = K * 4, ldb = N * 4;
     const int k0 = split * k_len;
     // Buffer ranges end at A's row M and at B's last byte: rows of a partial
@@ -497,10 +495,8 @@ gemm_f64_dma_kernel(const double* __restrict__ A, const double* __restrict__ B, 
     const int tid = threadIdx.x, lane = tid & 63, grp = lane >> 4;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wm = wave / WGN, wn = wave % WGN;
-    const int split = splits > 1 ? (int)blockIdx.x % splits : 0;
-    const int tile = splits > 1 ? (int)blockIdx.x / splits : (int)blockIdx.x;
-    int tm, tn;
-    tile_coords(tile, tiles_m * tiles_n, tiles_m, tiles_n, kHpGroupM, &tm, &tn);
+    int tm, tn, split;
+    block_coords((int)blockIdx.x, tiles_m, tiles_n, splits, kHpGroupM, &tm, &tn, &split);
     const int lda = K * 8, ldb = N * 8;
     const int k0 = split * k_len;
     // Buffer ranges as in gemm_f32_dma_kernel: partial last tiles and a ragged K.

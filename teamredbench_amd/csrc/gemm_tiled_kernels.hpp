@@ -375,12 +375,8 @@ gemm_tiled_kernel(const unsigned char* __restrict__ A, const unsigned char* __re
     const int lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wm = wave / WGN, wn = wave % WGN;
-    // Block -> (tile, K split). With one split the tile index is the block
-    // index (XCD-grouped); with several, the splits of a tile are adjacent.
-    const int split = splits > 1 ? (int)blockIdx.x % splits : 0;
-    const int tile = splits > 1 ? (int)blockIdx.x / splits : (int)blockIdx.x;
-    int tm, tn;
-    tile_coords(tile, tiles_m * tiles_n, tiles_m, tiles_n, group_m, &tm, &tn);
+    int tm, tn, split;
+    block_coords((int)blockIdx.x, tiles_m, tiles_n, splits, group_m, &tm, &tn, &split);
     // lda, ldb: bytes per A and B row; ldp: columns per row of a partial plane.
     const int k0 = split * k_len;  // first K element of this block
 
@@ -766,10 +762,8 @@ gemm_fp8_mi16_kernel(const unsigned char* __restrict__ A, const unsigned char* _
     const int g = lane >> 4, l16 = lane & 15;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wm = wave / WGN, wn = wave % WGN;
-    const int split = splits > 1 ? (int)blockIdx.x % splits : 0;
-    const int tile = splits > 1 ? (int)blockIdx.x / splits : (int)blockIdx.x;
-    int tm, tn;
-    tile_coords(tile, tiles_m * tiles_n, tiles_m, tiles_n, group_m, &tm, &tn);
+    int tm, tn, split;
+    block_coords((int)blockIdx.x, tiles_m, tiles_n, splits, group_m, &tm, &tn, &split);
     const int k0 = split * k_len;
 
     const int a_rows = min(BM, M - tm * BM);
