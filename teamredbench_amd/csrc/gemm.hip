@@ -23,7 +23,7 @@ int gemm_plan(int dtype, int64_t M, int64_t N, int64_t K, const DeviceProps& pro
         gemm_gemv_plan(dtype, M, N, K, props, plan) == MB_OK)
         return MB_OK;
     const char* why = "forced by the gemm_force_generic override";
-    if (!generic_only && gemm_tiled_plan(dtype, M, N, K, props, plan, &why) == MB_OK) return MB_OK;
+    if (!generic_only && gemm_tiled_plan(dtype, M, N, K, props, scratch, plan, &why) == MB_OK) return MB_OK;
     const int64_t grain = is_fp8(dtype) ? 16 : 8;
     const bool off16 = N % grain != 0 || K % grain != 0;
     const int rc = !generic_only && off16 && (gemm_strip_plan(dtype, M, N, K, props, scratch, plan) == MB_OK ||

@@ -4,11 +4,67 @@
 
 namespace mb {
 
+namespace {
+
+// Estimated time (us) of a plan: `blocks` blocks of configuration c, `stages` K
+// stages each, `bytes` of A, B and C, `feed` bytes of A and B into the blocks'
+// LDS, `outputs` elements of C.
+//   loop     rounds of blocks, the last one weighed by how full it is (idle CUs
+//            leave clock and bandwidth to the busy ones), each a block's stages
+//            plus its prologue and epilogue;
+//   stream   the operands from HBM, at a rate of the configuration's rows of B;
+//   feed     the panels that several blocks read, from the caches;
+//   splits   the reduction's launch, the partials written and read back.
+// The constants fit 10596 timings on MI355X (bf16, fp16, fp8; 300 random shapes
+// of M 1..8192, N and K 512..16384, every configuration, 15 split counts), the
+// near-best plans of a shape weighing most: 12% rms.
+struct TiledLoad {
+    double bytes, feed, outputs, cus;
+};
+
+double tiled_reduce_us(int splits, double outputs) {
+    constexpr double kReduce = 2.203, kPartialTBs = 5.142;
+    return splits > 1 ? kReduce + splits * outputs * 8.0 / (kPartialTBs * 1e6) : 0.0;
+}
+
+// Estimates that cannot come below `limit` end early.
+double tiled_estimate_us(int64_t e, int c, int64_t blocks, unsigned stages, int splits, const TiledLoad& load,
+                         double limit) {
+    // us per stage: 16-bit, fp8 16x16x128 (128 rows and more, an even stage count), fp8 32x32x64.
+    static constexpr double kStage[3][5] = {{0.705, 0.4243, 0.2606, 0.1358, 0.0836},
+                                            {0.6155, 0.3986, 0.2482, 0.0, 0.0},
+                                            {0.6778, 0.4372, 0.2759, 0.1403, 0.1067}};
+    static constexpr double kBlock[5] = {5.775, 2.869, 1.783, 1.158, 0.6144};      // us
+    static constexpr double kLastRound[5] = {0.672, 0.5805, 0.5087, 0.7886, 0.9845};  // nearly empty, of a full one
+    static constexpr double kStreamTBs[5] = {3.784, 6.407, 6.819, 5.621, 5.35};
+    constexpr double kLaunch = 2.478, kFeedTBs = 21.11;
+    const int cls = e == 2 ? 0 : c <= 2 && stages % 2 == 0 ? 1 : 2;
+    const double all = (double)blocks / load.cus, full = std::floor(all), part = all - full;
+    const double rounds = full + (part > 0.0 ? kLastRound[c] + (1.0 - kLastRound[c]) * part : 0.0);
+    const double bounds[3] = {rounds * ((double)stages * kStage[cls][c] + kBlock[c]),
+                              load.bytes / (kStreamTBs[c] * 1e6), load.feed / (kFeedTBs * 1e6)};
+    const double fixed = kLaunch + tiled_reduce_us(splits, load.outputs);
+    if (fixed + bounds[0] >= limit || fixed + bounds[1] >= limit) return limit;
+    double sum = 0.0;
+    for (double t : bounds) sum += t * t * t * t;   // the largest, the others showing where they come near
+    return fixed + std::sqrt(std::sqrt(sum));
+}
+
+constexpr int64_t kSplitCounts[] = {1, 2, 3, 4, 5, 6, 7, 8, 10, 12, 14, 16, 20, 24, 28, 32};
+
+// How much of the rules' estimated time another plan may take to replace it. At
+// 0.91, of the 300 shapes 61 ran more than 1% faster and 6 more than 2% slower
+// (7% at most), 1.056x in geometric mean over all; at 0.95 1.063x, but 10
+// slower, by up to 10%.
+constexpr double kMargin = 0.9;
+
+}  // namespace
+
 // Picks the tiled configuration for a shape, or returns MB_ERR_SHAPE with
 // *why set when the shape does not divide into any of them (or its buffers
 // need offsets beyond the 32-bit range of buffer addressing).
 int gemm_tiled_plan(int dtype, int64_t M, int64_t N, int64_t K, const DeviceProps& props,
-                    GemmPlan* plan, const char** why) {
+                    size_t scratch, GemmPlan* plan, const char** why) {
     const int64_t e = is_fp8(dtype) ? 1 : 2;
     const int64_t stage_k = kStageK / e;
     // B's rows must start on 16 bytes (N a multiple of 8, or of 16 for fp8)
@@ -47,6 +103,12 @@ int gemm_tiled_plan(int dtype, int64_t M, int64_t N, int64_t K, const DeviceProp
     auto split_ok = [&](int64_t sp) {
         if (!ragged_k) return K % (stage_k * sp) == 0;
         return sp <= stages && ((stages + sp - 1) / sp * sp * stage_k * N + 256) * e < (int64_t(1) << 31);
+    };
+    // Any other count whose last split still holds a stage (the kernels for a
+    // ragged K run it, the A pieces past K being zeros).
+    auto uneven_ok = [&](int64_t sp) {
+        const int64_t per = (stages + sp - 1) / sp;
+        return (sp - 1) * per < stages && (per * sp * stage_k * N + 256) * e < (int64_t(1) << 31);
     };
     auto split_k_len = [&](int64_t sp) { return (stages + sp - 1) / sp * stage_k; };
     const int64_t cus = props.cu_count > 0 ? props.cu_count : 256;
@@ -153,8 +215,52 @@ int gemm_tiled_plan(int dtype, int64_t M, int64_t N, int64_t K, const DeviceProp
             splits = s4;
         }
     }
+    // Those rules look at powers of two that divide K into whole stages, and at
+    // 256 x 256 tiles for whole panels of M only. A model of the measured times
+    // over every configuration and split count replaces their pick where it
+    // expects another to take less than kMargin of the time.
     const int64_t force_splits = tuning(MB_TUNE_GEMM_SPLITS);
-    if (force_splits >= 1 && split_ok(force_splits)) splits = (int)force_splits;
+    // A plan that fills the CUs exactly once stays (fp8 128 x 8192 x 8192: 25.2 us
+    // on 128 x 128 tiles at 4 splits, 28.0 on 64 x 128 at 2).
+    const int64_t rules_blocks = tiles(cfg) * splits;
+    if (pinned < 0 && force_splits < 1 && !fill_rule && (splits == 1 || rules_blocks != cus)) {
+        const double a_bytes = (double)(M * K * e), b_bytes = (double)(K * N * e), outputs = (double)(M * N);
+        auto estimate = [&](int c, int64_t tiles_m, int64_t tiles_n, int64_t sp, double limit) {
+            const TiledLoad load{a_bytes + b_bytes + 2.0 * outputs, (double)tiles_m * b_bytes + (double)tiles_n * a_bytes,
+                                 outputs, (double)cus};
+            return tiled_estimate_us(e, c, tiles_m * tiles_n * sp, (unsigned)(stages + sp - 1) / (unsigned)sp, (int)sp, load,
+                                     limit);
+        };
+        auto partials = [&](int64_t sp) { return sp > 1 ? (size_t)(sp * M * N) * sizeof(float) : 0; };
+        int best_cfg = cfg;
+        int64_t best_splits = splits;
+        double best = kMargin * estimate(cfg, (M + kConfigs[cfg].bm - 1) / kConfigs[cfg].bm,
+                                         (N + kConfigs[cfg].bn - 1) / kConfigs[cfg].bn, splits, 1e30);
+        for (int c = n128_only ? 2 : 0; c < 5; ++c) {
+            // fp8 rows of 64 bytes stream a wide B poorly: e5m2 7 x 13568 x 2560
+            // 11.8 us unsplit on 64 x 64 tiles, 9.7 on 64 x 128 at 2 splits.
+            if (c == 4 && e == 1 && N > 8192) continue;
+            const int64_t tm = (M + kConfigs[c].bm - 1) / kConfigs[c].bm, tn = (N + kConfigs[c].bn - 1) / kConfigs[c].bn;
+            for (int64_t sp : kSplitCounts) {
+                // More splits only add partials: past a round of blocks, or once
+                // the reduction alone takes what is left, no more of them.
+                if (sp > 1 && (c == 0 || 4 * tm * tn * sp > 5 * cus || tiled_reduce_us((int)sp, outputs) >= best)) break;
+                // Fewer blocks than 0.7 of the CUs keep too little in flight: e4m3
+                // 11 x 16064 x 3968 18.5 us on 126 blocks, 14.8 on 252.
+                const int64_t blocks = tm * tn * sp;
+                if (10 * blocks < 7 * cus && blocks < rules_blocks) continue;
+                const double t = estimate(c, tm, tn, sp, best);
+                if (t < best && uneven_ok(sp)) best = t, best_cfg = c, best_splits = sp;
+            }
+        }
+        // A call whose workspace would not hold the new plan's partials keeps
+        // the rules' plan; one that lacks a workspace the rules' plan needs is
+        // served from the library's own array, or refused, under either.
+        const size_t held = partials(splits), own = (size_t)MB_NOALLOC_SCRATCH_BYTES;
+        const size_t limit = scratch < held && held <= own ? own : scratch;
+        if (partials(best_splits) <= limit) cfg = best_cfg, splits = (int)best_splits;
+    }
+    if (force_splits >= 1 && (split_ok(force_splits) || uneven_ok(force_splits))) splits = (int)force_splits;
     if (kConfigs[cfg].bm > 128) splits = 1;   // the 256-row kernels carry no split path
     if (tiles(cfg) * splits > INT32_MAX) {
         *why = "more than 2^31 tiles";

@@ -142,6 +142,44 @@ def test_ragged_k_with_k_splits(lib, tune, dtype, config, splits, shape):
     assert info["implementation"] in PIPELINED and info["split_k"] == splits, info
 
 
+# Whole-stage K in parts that are not equal: the last split ends with K (shorter, one stage, odd and even counts).
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("config", [1, 2, 3, 4])
+@pytest.mark.parametrize("splits, stages", [(2, 13), (3, 13), (5, 13), (7, 20), (4, 10)])
+def test_unequal_k_splits(lib, tune, dtype, config, splits, stages):
+    tune(gemm_tiled_config=config, gemm_splits=splits)
+    k = stages * (64 if dtype.startswith("float8") else 32)
+    info = run_checked(lib, dtype, 200, 528, k, seed=10 * splits + config)
+    assert info["implementation"] in PIPELINED and info["split_k"] == splits, info
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("shape", [(9, 4688, 14112), (98, 4080, 3680), (25, 6208, 11456)])
+def test_optional_k_splits_without_a_workspace(lib, dtype, shape):
+    # K halves into whole stages once or not at all here, so the plan splits it unequally. A call that passes no
+    # workspace runs unsplit where equal parts were never to be had, or is refused as needing one.
+    m, n, k = shape
+    dt = capi.DTYPES[dtype]
+    run_checked(lib, dtype, *shape, seed=m)
+    ops = rp.gemm_inputs(m, n, k, dtype, seed=m)
+    da, db = ops["a"].cuda(), ops["b"].cuda()
+    out = torch.full((m * n + GUARD,), float("nan"), dtype=rp.gemm_output_dtype(dtype), device="cuda")
+    try:
+        lib.gemm(dt, da.data_ptr(), db.data_ptr(), out.data_ptr(), m, n, k, ops["scale_a"], ops["scale_b"], None, 0,
+                 torch.cuda.current_stream().cuda_stream)
+    except capi.NativeLibraryError as err:
+        assert err.status == capi.MB_ERR_WORKSPACE and (shape != (9, 4688, 14112) or dtype.startswith("float8")), err
+        return
+    torch.cuda.synchronize()
+    assert torch.isnan(out[m * n:].float()).all(), "the GEMM wrote past the end of C"
+    rows = sorted({0, m // 2, m - 1})
+    a64, b64 = ops["a"][rows].double().numpy(), ops["b"].double().numpy()
+    scale = float(ops["scale_a"]) * float(ops["scale_b"])
+    ref = scale * (a64 @ b64)
+    got = out[: m * n].view(m, n)[rows].cpu().double().numpy()
+    assert (np.abs(got - ref) <= elementwise_bound(dtype, k, np.abs(ref), scale * (np.abs(a64) @ np.abs(b64)))).all()
+
+
 GENERIC = "gfx950_mfma_generic"
 # (dtype, (M, N, K)): B rows off 16 bytes, or A rows off 16 bytes (K not a multiple of 8 / 16).
 FALLBACKS = [
