@@ -697,16 +697,17 @@ HighpChoice highp_choose(bool f64, int64_t M, int64_t N, int64_t K, int cus, siz
         return ch;
     }
     const int64_t e = f64 ? 8 : 4;
-    // Bytes of B up to a split's last stage and a partial tile's columns, and of an A panel.
     auto k_len = [&](int c, int64_t sp) {   // K per split, whole stages
         const int64_t stage_k = kHighpTiles[c].row / e, stages = (K + stage_k - 1) / stage_k;
         return (stages + sp - 1) / sp * stage_k;
     };
-    auto fits = [&](int64_t sp) {
-        const int64_t k_end = k_len(4, sp) * sp;   // the longest stages
+    // 32-bit offsets: bytes of B up to tile c's last stage of the last split (whole stages, so up to 128
+    // bytes of K past K itself) and a partial tile's columns, and of an A panel.
+    auto fits = [&](int c, int64_t sp) {
+        const int64_t k_end = k_len(c, sp) * sp;
         return (k_end * N + 256) * e < (int64_t(1) << 31) && 256 * k_end * e < (int64_t(1) << 31);
     };
-    if (!fits(1)) {
+    if (!fits(2, 1)) {   // 64-byte stages end nearest to K
         *why = "operand offsets exceed 32-bit buffer addressing (K*N or 256*K bytes >= 2 GiB)";
         return ch;
     }
@@ -747,7 +748,7 @@ HighpChoice highp_choose(bool f64, int64_t M, int64_t N, int64_t K, int cus, siz
     // 128-byte rows of A (2048^3 249 against 254 us; with more blocks their
     // 128 KiB of ring leave one block per CU and run 8-9% slower).
     if ((M % 128 == 0 && N % 128 == 0 && tiles(2) % cus == 0) || (K < 128 && M >= 512)) {
-        ch.config = f64 && tiles(2) <= cus && K >= 128 ? 3 : 2;
+        ch.config = f64 && tiles(2) <= cus && K >= 128 && fits(3, 1) ? 3 : 2;
         return ch;
     }
     // The rest: the tile and the K split that a cost model rates fastest,
@@ -775,8 +776,8 @@ HighpChoice highp_choose(bool f64, int64_t M, int64_t N, int64_t K, int cus, siz
         const int c = kTiles[i];
         for (const int sp : kSplits) {
             const int64_t blocks = tiles(c) * sp, kl = k_len(c, sp);
-            if (sp > 1 && (K < 64 * sp || kl * (sp - 1) >= K || 4 * cus < blocks || !fits(sp) ||
-                           (size_t)(sp * M * N * e) > scratch))
+            if (!fits(c, sp) || (sp > 1 && (K < 64 * sp || kl * (sp - 1) >= K || 4 * cus < blocks ||
+                                            (size_t)(sp * M * N * e) > scratch)))
                 continue;
             const double r = (double)rounds(blocks), used = blocks < cus ? (double)blocks / (double)cus : 1.0;
             const double eff = kEff[i] * (c != 2 && blocks <= cus ? 0.89 : c == 5 && blocks > 2 * cus ? 0.83 : 1.0);
@@ -788,12 +789,14 @@ HighpChoice highp_choose(bool f64, int64_t M, int64_t N, int64_t K, int cus, siz
         }
     }
     // fp64 alone on a CU: 128-byte rows of A (above).
-    if (f64 && ch.config == 2 && tiles(2) * ch.splits <= cus && k_len(3, ch.splits) * (ch.splits - 1) < K) ch.config = 3;
+    if (f64 && ch.config == 2 && tiles(2) * ch.splits <= cus && k_len(3, ch.splits) * (ch.splits - 1) < K &&
+        fits(3, ch.splits))
+        ch.config = 3;
     // One unsplit round of at least six 128-row panels runs 128 x 32 tiles:
     // 128-row tiles without a workspace are what a plan of 1000^3 has always
     // reported (26.7 us fp32 and 41.9 fp64, against 65 and 123 on 128 x 128;
     // 64 x 64 tiles take 21.8 and 39.0).
-    if (ch.splits == 1 && ch.config != 2 && M >= 768 && tiles(4) <= cus) ch.config = 6;
+    if (ch.splits == 1 && ch.config != 2 && M >= 768 && tiles(4) <= cus && fits(6, 1)) ch.config = 6;
     return ch;
 }
 
