@@ -115,7 +115,9 @@ int mb_time_stream(int op, int dtype, void* dst, const void* b, const void* c,
  * be NULL when that size is 0). The kernels leave it in a state the next
  * call can use without clearing. FLOAT32 / FLOAT64 (K split over idle CUs) and
  * the other types with rows off 16 bytes (operands repacked, or K split) use it only to run
- * faster: with less than that size, or NULL, they run without.
+ * faster: with less than that size, NULL, or an address off 16 bytes, they run
+ * without. A workspace off 16 bytes must still have that size where the type
+ * and shape need one.
  */
 int mb_gemm(int dtype, const void* A, const void* B, void* C, int64_t M,
             int64_t N, int64_t K, float scale_a, float scale_b, void* workspace,

@@ -130,8 +130,8 @@ int check_gemm_args(int dtype, const void* A, const void* B, void* C, int64_t M,
     return MB_OK;
 }
 
-size_t scratch_given(const void* workspace, size_t workspace_bytes) {
-    return workspace != nullptr ? workspace_bytes : 0;
+Scratch scratch_given(const void* workspace, size_t workspace_bytes) {
+    return Scratch{workspace != nullptr ? workspace_bytes : 0, (reinterpret_cast<uintptr_t>(workspace) & 15u) == 0};
 }
 
 // Event-timed loop shared by the mb_time_* entry points.
@@ -366,7 +366,7 @@ size_t mb_gemm_workspace_size(int dtype, int64_t M, int64_t N, int64_t K) {
     const DeviceProps* props = nullptr;
     if (current_device_props(&props) != MB_OK) return 0;
     GemmPlan plan;
-    if (gemm_plan(dtype, M, N, K, *props, SIZE_MAX, &plan) != MB_OK) return 0;
+    if (gemm_plan(dtype, M, N, K, *props, Scratch{SIZE_MAX}, &plan) != MB_OK) return 0;
     return plan.workspace;
 }
 
@@ -392,7 +392,7 @@ int mb_gemm_noalloc(int dtype, const void* A, const void* B, void* C, int64_t M,
     if (rc != MB_OK) return rc;
     GemmPlan plan;
     // No scratch for plans that can do without: those calls may overlap on one GPU.
-    if ((rc = gemm_plan(dtype, M, N, K, *props, 0, &plan)) != MB_OK) return rc;
+    if ((rc = gemm_plan(dtype, M, N, K, *props, Scratch{0}, &plan)) != MB_OK) return rc;
     if (plan.workspace > (size_t)MB_NOALLOC_SCRATCH_BYTES) {
         set_error("GEMM %s %lldx%lldx%lld needs %zu scratch bytes; mb_gemm_noalloc holds %zu "
                   "(use mb_gemm with a caller workspace)",
@@ -480,7 +480,7 @@ int mb_kernel_info(int kind, int a, int b, int64_t m, int64_t n, int64_t k, char
     }
     if (kind == MB_KIND_GEMM) {
         GemmPlan plan;
-        if ((rc = gemm_plan(a, m, n, k, *props, SIZE_MAX, &plan)) != MB_OK) return rc;
+        if ((rc = gemm_plan(a, m, n, k, *props, Scratch{SIZE_MAX}, &plan)) != MB_OK) return rc;
         j.str("implementation", plan.implementation);
         j.num("threads_per_block", plan.threads);
         j.num("grid_blocks", plan.grid);

@@ -4,7 +4,7 @@
 
 namespace mb {
 
-int gemm_plan(int dtype, int64_t M, int64_t N, int64_t K, const DeviceProps& props, size_t scratch,
+int gemm_plan(int dtype, int64_t M, int64_t N, int64_t K, const DeviceProps& props, Scratch scratch,
               GemmPlan* plan) {
     if (dtype != MB_DT_BFLOAT16 && dtype != MB_DT_FLOAT16 && !is_fp8(dtype) && dtype != MB_DT_FLOAT32 &&
         dtype != MB_DT_FLOAT64) {
@@ -17,7 +17,8 @@ int gemm_plan(int dtype, int64_t M, int64_t N, int64_t K, const DeviceProps& pro
                   (long long)K);
         return MB_ERR_INVALID_ARG;
     }
-    if (dtype == MB_DT_FLOAT32 || dtype == MB_DT_FLOAT64) return gemm_highp_plan(dtype, M, N, K, props, scratch, plan);
+    const size_t optional = scratch.on_16 ? scratch.bytes : 0;
+    if (dtype == MB_DT_FLOAT32 || dtype == MB_DT_FLOAT64) return gemm_highp_plan(dtype, M, N, K, props, optional, plan);
     const bool generic_only = tuning(MB_TUNE_GEMM_FORCE_GENERIC) == 1;
     if (!generic_only && tuning(MB_TUNE_GEMM_NO_SMALL_M) != 1 &&
         gemm_gemv_plan(dtype, M, N, K, props, plan) == MB_OK)
@@ -26,8 +27,8 @@ int gemm_plan(int dtype, int64_t M, int64_t N, int64_t K, const DeviceProps& pro
     if (!generic_only && gemm_tiled_plan(dtype, M, N, K, props, scratch, plan, &why) == MB_OK) return MB_OK;
     const int64_t grain = is_fp8(dtype) ? 16 : 8;
     const bool off16 = N % grain != 0 || K % grain != 0;
-    const int rc = !generic_only && off16 && (gemm_strip_plan(dtype, M, N, K, props, scratch, plan) == MB_OK ||
-                                              gemm_packed_plan(dtype, M, N, K, props, scratch, plan) == MB_OK)
+    const int rc = !generic_only && off16 && (gemm_strip_plan(dtype, M, N, K, props, optional, plan) == MB_OK ||
+                                              gemm_packed_plan(dtype, M, N, K, props, optional, plan) == MB_OK)
                        ? MB_OK : gemm_generic_plan(dtype, M, N, K, plan);
     plan->fallback = why;
     return rc;

@@ -87,7 +87,7 @@ int gemm_packed_plan(int dtype, int64_t M, int64_t N, int64_t K, const DevicePro
     const int64_t np = (N + grain - 1) / grain * grain, kp = (K + grain - 1) / grain * grain;
     GemmPlan p;
     const char* why = "";
-    if (gemm_tiled_plan(dtype, M, np, kp, props, SIZE_MAX, &p, &why) != MB_OK) return MB_ERR_SHAPE;
+    if (gemm_tiled_plan(dtype, M, np, kp, props, Scratch{SIZE_MAX}, &p, &why) != MB_OK) return MB_ERR_SHAPE;
     p.pack_a = kp != K;
     p.pack_b = np != N;
     // Rows on 128 bytes: whole cache lines per tile row.

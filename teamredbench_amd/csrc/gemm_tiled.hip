@@ -64,7 +64,7 @@ constexpr double kMargin = 0.9;
 // *why set when the shape does not divide into any of them (or its buffers
 // need offsets beyond the 32-bit range of buffer addressing).
 int gemm_tiled_plan(int dtype, int64_t M, int64_t N, int64_t K, const DeviceProps& props,
-                    size_t scratch, GemmPlan* plan, const char** why) {
+                    Scratch scratch, GemmPlan* plan, const char** why) {
     const int64_t e = is_fp8(dtype) ? 1 : 2;
     const int64_t stage_k = kStageK / e;
     // B's rows must start on 16 bytes (N a multiple of 8, or of 16 for fp8)
@@ -223,7 +223,8 @@ int gemm_tiled_plan(int dtype, int64_t M, int64_t N, int64_t K, const DeviceProp
     // A plan that fills the CUs exactly once stays (fp8 128 x 8192 x 8192: 25.2 us
     // on 128 x 128 tiles at 4 splits, 28.0 on 64 x 128 at 2).
     const int64_t rules_blocks = tiles(cfg) * splits;
-    if (pinned < 0 && force_splits < 1 && !fill_rule && (splits == 1 || rules_blocks != cus)) {
+    // (An unsplit pick stays with a workspace off 16 bytes, which it leaves alone.)
+    if (pinned < 0 && force_splits < 1 && !fill_rule && (splits == 1 ? scratch.on_16 : rules_blocks != cus)) {
         const double a_bytes = (double)(M * K * e), b_bytes = (double)(K * N * e), outputs = (double)(M * N);
         auto estimate = [&](int c, int64_t tiles_m, int64_t tiles_n, int64_t sp, double limit) {
             const TiledLoad load{a_bytes + b_bytes + 2.0 * outputs, (double)tiles_m * b_bytes + (double)tiles_n * a_bytes,
@@ -257,7 +258,7 @@ int gemm_tiled_plan(int dtype, int64_t M, int64_t N, int64_t K, const DeviceProp
         // the rules' plan; one that lacks a workspace the rules' plan needs is
         // served from the library's own array, or refused, under either.
         const size_t held = partials(splits), own = (size_t)MB_NOALLOC_SCRATCH_BYTES;
-        const size_t limit = scratch < held && held <= own ? own : scratch;
+        const size_t limit = scratch.bytes < held && held <= own ? own : scratch.bytes;
         if (partials(best_splits) <= limit) cfg = best_cfg, splits = (int)best_splits;
     }
     if (force_splits >= 1 && (split_ok(force_splits) || uneven_ok(force_splits))) splits = (int)force_splits;

@@ -131,10 +131,17 @@ struct GemmPlan {
     int config = 0;             // configuration within the family
 };
 
-// `scratch`: the largest workspace the caller can give to plans that use one
-// only to run faster (a caller that gives none still gets a plan without it).
+// The workspace a caller gives: its bytes, and whether it starts on 16 bytes.
+struct Scratch {
+    size_t bytes = 0;
+    bool on_16 = true;
+};
+
+// `scratch`: what there is for plans that use a workspace only to run faster
+// (with too little, or one off 16 bytes, they make do without: repacked
+// operands are LDS-DMA sources, and partials are stored 16 bytes at a time).
 // Plans that cannot do without a workspace ask for it whatever `scratch` is.
-int gemm_plan(int dtype, int64_t M, int64_t N, int64_t K, const DeviceProps& props, size_t scratch,
+int gemm_plan(int dtype, int64_t M, int64_t N, int64_t K, const DeviceProps& props, Scratch scratch,
               GemmPlan* plan);
 
 // One launch of the MFMA-only kernel of instruction `kind` (MB_MFMA_*).

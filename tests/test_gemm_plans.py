@@ -28,15 +28,15 @@ class Plan(NamedTuple):
 
 @pytest.fixture(scope="session")
 def plans(tmp_path_factory):
-    """plans([(dtype name, M, N, K, scratch bytes), ...]) -> [Plan, ...]"""
+    """plans([(dtype name, M, N, K, scratch bytes), ...], on_16=scratch starts on 16 bytes) -> [Plan, ...]"""
     compiler = shutil.which("amdclang++") or "/opt/rocm/bin/amdclang++"
     exe = tmp_path_factory.mktemp("plans") / "gemm_plan_host"
     lib = build.library_path()
     subprocess.run([compiler, "-O1", "-std=c++20", "-D__HIP_PLATFORM_AMD__", "-I/opt/rocm/include",
                     str(TESTS / "gemm_plan_host.cpp"), str(lib), f"-Wl,-rpath,{lib.parent}", "-o", str(exe)], check=True)
 
-    def ask(shapes):
-        lines = "".join(f"{capi.DTYPES[dtype]} {m} {n} {k} {scratch}\n" for dtype, m, n, k, scratch in shapes)
+    def ask(shapes, on_16=True):
+        lines = "".join(f"{capi.DTYPES[dtype]} {m} {n} {k} {scratch} {int(on_16)}\n" for dtype, m, n, k, scratch in shapes)
         out = subprocess.run([str(exe)], input=lines, capture_output=True, text=True, check=True).stdout.splitlines()
         assert len(out) == len(shapes)
         rows = [line.split() for line in out]
@@ -78,3 +78,31 @@ def test_full_precision_offsets_stay_in_31_bits(plans, dtype):
         assert plan.tile_m * end * size < LIMIT, (m, n, k, scratch, plan)
         assert (plan.split_k - 1) * per * plan.tile_k < k, "a split without a stage"
     assert ring > len(shapes) // 2
+
+
+OFF_16_WORKSPACE = [
+    ("bfloat16", 300, 513, 512), ("float8_e4m3fn", 300, 1031, 1029), ("float16", 40, 2047, 4099),   # repacked, few rows
+    ("float32", 5, 4099, 2051), ("float64", 600, 704, 1904), ("float32", 1000, 1500, 2000),          # K splits
+    ("bfloat16", 25, 208, 3552), ("float16", 6, 400, 2240),     # K splits that the equal parts of K do not give
+]
+
+
+def test_a_workspace_off_16_bytes_is_as_none_where_it_is_optional(plans):
+    given = [shape + (EVERYTHING,) for shape in OFF_16_WORKSPACE]
+    assert all(plan.workspace > 0 for plan in plans(given))
+    assert plans(given, on_16=False) == plans([shape + (0,) for shape in OFF_16_WORKSPACE])
+    # Where a plan cannot do without, it asks for the same bytes at any address.
+    needed = [("float16", 16, 8192, 8192), ("bfloat16", 1, 4096, 4096)]
+    assert plans([s + (EVERYTHING,) for s in needed], on_16=False) == plans([s + (EVERYTHING,) for s in needed])
+
+
+def test_the_reported_workspace_size_is_enough_at_any_address(plans):
+    rng = random.Random(16)
+    shapes = [(rng.choice(("bfloat16", "float16", "float8_e4m3fn", "float32", "float64")), int(2048 ** rng.random()),
+               int(8 * 1024 ** rng.random()), int(8 * 1024 ** rng.random())) for _ in range(3000)]
+    shapes += [(dtype, m, n // 16 * 16 + 16, k // 16 * 16 + 16) for dtype, m, n, k in shapes]
+    sizes = [plan.workspace for plan in plans([shape + (EVERYTHING,) for shape in shapes])]
+    exact = [shape + (size,) for shape, size in zip(shapes, sizes)]
+    for on_16 in (True, False):
+        for shape, size, plan in zip(shapes, sizes, plans(exact, on_16=on_16)):
+            assert plan.workspace <= size, (shape, size, on_16, plan)

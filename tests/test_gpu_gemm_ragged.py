@@ -180,6 +180,37 @@ def test_optional_k_splits_without_a_workspace(lib, dtype, shape):
     assert (np.abs(got - ref) <= elementwise_bound(dtype, k, np.abs(ref), scale * (np.abs(a64) @ np.abs(b64)))).all()
 
 
+# A workspace off 16 bytes: operands repacked into it would not be LDS-DMA sources, so calls that can do without it
+# leave it alone; a plan that needs its K splits runs them there.
+@pytest.mark.parametrize("offset", [4, 8])
+@pytest.mark.parametrize("dtype, shape, uses_it", [
+    ("bfloat16", (300, 513, 512), False), ("float8_e4m3fn", (300, 1031, 1029), False),
+    ("float16", (40, 2047, 4099), False), ("float32", (5, 4099, 2051), False), ("float64", (600, 704, 1904), False),
+    ("bfloat16", (25, 208, 3552), False), ("float16", (16, 8192, 8192), True)])
+def test_workspace_off_16_bytes(lib, dtype, shape, uses_it, offset):
+    m, n, k = shape
+    dt = capi.DTYPES[dtype]
+    ops = rp.gemm_inputs(m, n, k, dtype, seed=m + offset)
+    da, db = ops["a"].cuda(), ops["b"].cuda()
+    tdt = ops["a"].dtype if dtype in ("float32", "float64") else rp.gemm_output_dtype(dtype)
+    out = torch.full((m * n + GUARD,), float("nan"), dtype=tdt, device="cuda")
+    size = lib.gemm_workspace_size(dt, m, n, k)
+    assert size > 0
+    ws = torch.full((size + offset + GUARD,), 0x7F, dtype=torch.uint8, device="cuda")
+    lib.gemm(dt, da.data_ptr(), db.data_ptr(), out.data_ptr(), m, n, k, ops["scale_a"], ops["scale_b"],
+             ws.data_ptr() + offset, size, torch.cuda.current_stream().cuda_stream)
+    torch.cuda.synchronize()
+    assert torch.isnan(out[m * n:].float()).all(), "the GEMM wrote past the end of C"
+    assert (ws[:offset] == 0x7F).all() and (ws[offset + size:] == 0x7F).all()
+    assert uses_it or (ws == 0x7F).all(), "the GEMM used a workspace off 16 bytes"
+    rows = sorted({0, m // 2, m - 1})
+    a64, b64 = ops["a"][rows].double().numpy(), ops["b"].double().numpy()
+    scale = float(ops["scale_a"]) * float(ops["scale_b"])
+    ref = scale * (a64 @ b64)
+    got = out[: m * n].view(m, n)[rows].cpu().double().numpy()
+    assert (np.abs(got - ref) <= elementwise_bound(dtype, k, np.abs(ref), scale * (np.abs(a64) @ np.abs(b64)))).all()
+
+
 GENERIC = "gfx950_mfma_generic"
 # (dtype, (M, N, K)): B rows off 16 bytes, or A rows off 16 bytes (K not a multiple of 8 / 16).
 FALLBACKS = [
