@@ -184,7 +184,7 @@ template <> struct BitsOf<4> { typedef uint32_t T; };
 template <> struct BitsOf<8> { typedef uint64_t T; };
 
 template <int OP, int DT>
-__device__ inline void scalar_element(void* dst, const void* b, const void* c, uint64_t i,
+__device__ inline void scalar_element(void* dst, const void* b, const void* c, int64_t i,
                                       float s, double sd) {
     typedef typename Scalar<DT>::T T;
     const T* B = static_cast<const T*>(b);
@@ -220,16 +220,20 @@ __device__ inline void store_chunk(u32x4_any* p, u32x4 v) {
     }
 }
 
-// Vector body over `chunks` 16-byte chunks that start `head` elements into
-// the arrays, then the `edge` elements outside it (a head of less than a
-// 128-byte line, a tail of less than a chunk) by the grid's first threads.
+// Vector body over the `chunks` 16-byte chunks that start at dst, b and c, then
+// the `edge` elements outside it (`head` of them before the pointers, less than
+// a 128-byte line; a tail of less than a chunk) by the grid's first threads.
 // span == 0: grid-stride -- consecutive trips of a thread are one grid apart.
 // span  > 0: each block walks its own contiguous run of `span` chunks, the
 //            block's lanes side by side, trips one block-width apart.
 // Chunks need no alignment: gfx950 loads and stores 16 bytes at any address
 // (u32x4_any), with the instructions it uses for aligned ones. The plan picks
 // `head` so that dst's chunks are aligned; b and c then start wherever they
-// do. Bound: HBM, as with aligned arrays. On MI355X, source one element off,
+// do. The host moves the pointers past the head, and `edge` is loaded beside
+// `chunks`, `head` by the edge's threads alone: shifts and a late argument
+// load in every wave cost aligned arrays 0.03-0.06 us (fp64 triad of 2^20
+// elements 5.39 us, 5.33 so; fp32 triad of 2^22 4.12, 4.07).
+// Bound: HBM, as with aligned arrays. On MI355X, source one element off,
 // against one element per lane and load (the kernel such arrays had before):
 // fp16 copy of 5e7 elements 294 -> 36 us (aligned 36), bf16 scale of 6e7 374
 // -> 43 (42), fp32 triad of 2e8 1490 -> 388 (381), int8 copy of 4e8 2240 ->
@@ -237,11 +241,11 @@ __device__ inline void store_chunk(u32x4_any* p, u32x4 v) {
 template <int OP, int DT, int U, bool NT>
 __global__ void __launch_bounds__(1024)
 stream_vec_kernel(void* __restrict__ dst, const void* __restrict__ b, const void* __restrict__ c,
-                  uint64_t chunks, unsigned head, unsigned edge, uint64_t span, float s, double sd) {
+                  uint64_t chunks, uint64_t edge, uint64_t span, float s, unsigned head, double sd) {
     constexpr int esize = (DT == MB_DT_FLOAT32) ? 4 : (DT == MB_DT_FLOAT64) ? 8 : (DT == MB_DT_INT8) ? 1 : 2;
-    const u32x4_any* B = reinterpret_cast<const u32x4_any*>(static_cast<const char*>(b) + head * esize);
-    const u32x4_any* C = reinterpret_cast<const u32x4_any*>(static_cast<const char*>(c) + head * esize);
-    u32x4_any* D = reinterpret_cast<u32x4_any*>(static_cast<char*>(dst) + head * esize);
+    const u32x4_any* B = static_cast<const u32x4_any*>(b);
+    const u32x4_any* C = static_cast<const u32x4_any*>(c);
+    u32x4_any* D = static_cast<u32x4_any*>(dst);
     const uint64_t tid = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
     uint64_t stride, end, i;
     if (span == 0) {
@@ -275,12 +279,15 @@ stream_vec_kernel(void* __restrict__ dst, const void* __restrict__ b, const void
         if (OP == MB_OP_TRIAD) vc = load_chunk<NT>(C + i);
         store_chunk<NT>(D + i, ChunkOp<OP, DT>::apply(vb, vc, s, sd));
     }
-    if (tid < edge) scalar_element<OP, DT>(dst, b, c, tid < head ? tid : chunks * (16 / esize) + tid, s, sd);
+    if (tid < edge) {
+        const int64_t i = (int64_t)tid - (int64_t)head;   // elements past dst
+        scalar_element<OP, DT>(dst, b, c, tid < head ? i : (int64_t)chunks * (16 / esize) + i, s, sd);
+    }
 }
 
 // ---- dispatch --------------------------------------------------------------
 
-typedef void (*VecKernel)(void*, const void*, const void*, uint64_t, unsigned, unsigned, uint64_t, float, double);
+typedef void (*VecKernel)(void*, const void*, const void*, uint64_t, uint64_t, uint64_t, float, unsigned, double);
 
 template <int OP, int DT>
 VecKernel pick_vec(int u, bool nt) {
@@ -402,12 +409,12 @@ int stream_plan(int op, int dtype, const void* dst, const void* b, const void* c
     // 235 us there and 198 here (fp32 copy of 1.5e8; aligned 193), 418 and
     // 384 (fp32 triad of 2e8), 150 and 128 (int8 copy of 4e8).
     constexpr uint64_t kLine = 128;
-    const uint64_t per_chunk = 16 / (uint64_t)esize;
-    const uint64_t to_boundary = (kLine - reinterpret_cast<uintptr_t>(dst) % kLine) % kLine;
-    const uint64_t head = to_boundary % (uint64_t)esize == 0 ? to_boundary / (uint64_t)esize : 0;
+    const int eshift = __builtin_ctz((unsigned)esize), per_chunk_shift = 4 - eshift;
+    const uint64_t to_boundary = -reinterpret_cast<uintptr_t>(dst) % kLine;
+    const uint64_t head = to_boundary % (uint64_t)esize == 0 ? to_boundary >> eshift : 0;
     plan->head = head < n ? head : n;
-    plan->chunks = (n - plan->head) / per_chunk;
-    plan->tail = n - plan->head - plan->chunks * per_chunk;
+    plan->chunks = (n - plan->head) >> per_chunk_shift;
+    plan->tail = n - plan->head - (plan->chunks << per_chunk_shift);
     uint64_t work_items = (plan->chunks + (uint64_t)u - 1) / (uint64_t)u;
     const uint64_t edge = plan->head + plan->tail;
     if (work_items < edge) work_items = edge;
@@ -438,8 +445,11 @@ int stream_launch(int op, int dtype, void* dst, const void* b, const void* c, ui
         set_error("no stream kernel for op %d dtype %d", op, dtype);
         return MB_ERR_UNSUPPORTED;
     }
-    hipLaunchKernelGGL(k, dim3(plan.blocks), dim3(plan.threads), 0, stream, dst, b, c, plan.chunks,
-                       (unsigned)plan.head, (unsigned)(plan.head + plan.tail), plan.span, sf, s);
+    const uint64_t shift = plan.head * (uint64_t)dtype_size(dtype);   // bytes of the head
+    hipLaunchKernelGGL(k, dim3(plan.blocks), dim3(plan.threads), 0, stream, static_cast<char*>(dst) + shift,
+                       static_cast<const char*>(b) + shift,
+                       c != nullptr ? static_cast<const char*>(c) + shift : nullptr, plan.chunks, plan.head + plan.tail,
+                       plan.span, sf, (unsigned)plan.head, s);
     MB_HIP_TRY(hipGetLastError());
     return MB_OK;
 }
