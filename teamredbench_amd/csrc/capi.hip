@@ -460,8 +460,8 @@ int mb_kernel_info(int kind, int a, int b, int64_t m, int64_t n, int64_t k, char
     Json j;
     if (kind == MB_KIND_STREAM) {
         const int op = a, dtype = b;
-        // Plan against 16-byte aligned buffers: the layout torch allocations have.
-        alignas(16) static char dummy[16];
+        // Plan against buffers on dst's 128-byte line (no head), as torch allocates them.
+        alignas(128) static char dummy[128];
         StreamPlan plan;
         if ((rc = stream_plan(op, dtype, dummy, dummy, dummy, (uint64_t)m, (int)n, *props, &plan)) !=
             MB_OK)

@@ -179,6 +179,16 @@ def test_kernel_info_keys(lib):
     assert info["arch"].startswith("gfx950")
 
 
+@pytest.mark.parametrize("mode, dtype, n, blocks", [
+    ("copy", "float32", 4096, 1), ("copy", "float32", 4100, 2), ("scale", "bfloat16", 8200, 2),
+    ("triad", "float64", 1024, 1), ("triad", "float64", 1026, 2), ("copy", "int8", 3 * 16384, 3)])
+def test_kernel_info_describes_allocations(lib, mode, dtype, n, blocks):
+    # The plan of arrays that start on a 128-byte line, as allocations do: 256 threads x 4 chunks of 16 bytes a block
+    # (2 for the triad), one block more for one chunk more.
+    info = lib.stream_info(capi.OPS[mode], capi.DTYPES[dtype], n)
+    assert info["grid_blocks"] == blocks, info
+
+
 @pytest.mark.parametrize("mode, dtype, n, nontemporal", [
     ("triad", "float32", 1 << 28, True),     # 3 GiB a pass: streams past the Infinity Cache
     ("triad", "float32", 1 << 24, False),    # 192 MiB: fits, ordinary accesses keep it there
