@@ -4,7 +4,8 @@
 // copies (their DMA loads need 16-byte sources; gemm_tiled_kernels.hpp, ANY_N).
 //
 // The copy is bound by HBM: it reads and writes each repacked operand once, a
-// small part of a product with many rows (up to 64 go to gemm_strip.hip).
+// small part of a product with many rows (up to 64 go to gemm_strip.hip) and a
+// long K; kPackMinK says from where on it pays.
 #include "gemm_common.hpp"
 
 namespace mb {
@@ -78,12 +79,23 @@ PackJob pack_job(const void* src, void* dst, int64_t rows, int64_t row_bytes, in
 
 size_t align256(size_t v) { return (v + 255) & ~size_t(255); }
 
+// The least K that pays for the copy and its launch (about 5 us together) against
+// the bounds-checked kernel, whose time grows with K; columns under one of its
+// tiles move its operands less often. 1800 random products on MI355X (M 1..8192,
+// N and K 1..4096, all four types): repacked from these K on, one ran slower than
+// on the bounds-checked kernel (0.96x) and all 1.28x faster in geometric mean;
+// repacked everywhere, 977 ran slower, by up to 2.3x (fp16 5776 x 407 x 96 7.3
+// against 14.7 us, e5m2 158 x 413 x 368 10.6 against 12.6 at worst beyond).
+constexpr int64_t kPackMinK = 256, kPackMinKNarrow = 320, kPackNarrowN = 128;
+
 }  // namespace
 
 int gemm_packed_plan(int dtype, int64_t M, int64_t N, int64_t K, const DeviceProps& props, size_t scratch,
                      GemmPlan* plan) {
     const int64_t e = is_fp8(dtype) ? 1 : 2, grain = 16 / e;
     if (N >= (int64_t(1) << 31) || K >= (int64_t(1) << 31) || M >= (int64_t(1) << 31)) return MB_ERR_SHAPE;
+    // (A forced tile is a call for these kernels.)
+    if (K < (N < kPackNarrowN ? kPackMinKNarrow : kPackMinK) && tuning(MB_TUNE_GEMM_TILED_CONFIG) < 0) return MB_ERR_SHAPE;
     const int64_t np = (N + grain - 1) / grain * grain, kp = (K + grain - 1) / grain * grain;
     GemmPlan p;
     const char* why = "";

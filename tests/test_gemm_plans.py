@@ -106,3 +106,14 @@ def test_the_reported_workspace_size_is_enough_at_any_address(plans):
     for on_16 in (True, False):
         for shape, size, plan in zip(shapes, sizes, plans(exact, on_16=on_16)):
             assert plan.workspace <= size, (shape, size, on_16, plan)
+
+
+# (M, N, K), repacked: rows off 16 bytes and more than 64 of them.
+@pytest.mark.parametrize("dtype", ["bfloat16", "float16", "float8_e4m3fn", "float8_e5m2"])
+@pytest.mark.parametrize("shape, repacked", [((4594, 13, 15), False), ((5776, 407, 97), False), ((205, 301, 193), False),
+                                             ((300, 129, 255), False), ((300, 129, 257), True), ((300, 127, 319), False),
+                                             ((300, 127, 321), True), ((8192, 50257, 4096), True)])
+def test_operands_are_repacked_where_it_pays(plans, dtype, shape, repacked):
+    # The bounds-checked kernel has two stages; the pipelined ones on repacked operands have more.
+    plan, = plans([(dtype, *shape, EVERYTHING)])
+    assert (plan.k_stages > 2 and plan.workspace > 0) is repacked, plan
