@@ -262,6 +262,11 @@ int launch_dt(const void* A, const void* B, void* C, int64_t M, int64_t N, int64
 int gemm_strip_plan(int dtype, int64_t M, int64_t N, int64_t K, const DeviceProps& props, size_t scratch,
                     GemmPlan* plan) {
     if (M < 1 || M > kStripMaxM) return MB_ERR_SHAPE;
+    // Under one step of K only the tail runs, which loads A element by element:
+    // three or four fragments of rows of a 16-bit type then take 5.1-6.5 us, the
+    // bounds-checked kernel 4.8-5.9 (139 products, 0.76-1.32x; from one step of K
+    // on 0.96-2.0x, fp8 1.0-2.4x but for one at 0.90, fewer rows 1.1-3.3x).
+    if (M > 32 && K < kStripStep && !is_fp8(dtype)) return MB_ERR_SHAPE;
     const int fm = (int)(M + 15) / 16;
     const int64_t e = is_fp8(dtype) ? 1 : 2, cols = strip_cols(dtype, fm);
     // 32-bit offsets within a step (32 rows of B) and 32-bit K and column indices.

@@ -117,3 +117,12 @@ def test_operands_are_repacked_where_it_pays(plans, dtype, shape, repacked):
     # The bounds-checked kernel has two stages; the pipelined ones on repacked operands have more.
     plan, = plans([(dtype, *shape, EVERYTHING)])
     assert (plan.k_stages > 2 and plan.workspace > 0) is repacked, plan
+
+
+@pytest.mark.parametrize("dtype, shape, few_rows", [
+    ("bfloat16", (33, 129, 31), False), ("float16", (64, 1031, 5), False), ("bfloat16", (32, 129, 31), True),
+    ("float16", (33, 129, 33), True), ("float8_e4m3fn", (64, 129, 31), True), ("bfloat16", (64, 8, 33), True)])
+def test_few_row_kernel_starts_at_a_step_of_k(plans, dtype, shape, few_rows):
+    # The few-row kernel's tiles are 128 K values deep, the bounds-checked kernel's one stage of 64 bytes.
+    plan, = plans([(dtype, *shape, EVERYTHING)])
+    assert (plan.tile_k == 128) is few_rows, plan
