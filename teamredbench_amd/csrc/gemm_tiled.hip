@@ -52,11 +52,24 @@ double tiled_estimate_us(int64_t e, int c, int64_t blocks, unsigned stages, int 
 
 constexpr int64_t kSplitCounts[] = {1, 2, 3, 4, 5, 6, 7, 8, 10, 12, 14, 16, 20, 24, 28, 32};
 
-// How much of the rules' estimated time another plan may take to replace it. At
-// 0.91, of the 300 shapes 61 ran more than 1% faster and 6 more than 2% slower
-// (7% at most), 1.056x in geometric mean over all; at 0.95 1.063x, but 10
-// slower, by up to 10%.
+// How much of the rules' estimated time another plan may take to replace it (what
+// it gives: below).
 constexpr double kMargin = 0.9;
+
+// Two kinds of plans run longer than the model says:
+// - a K split where the rules have none launches a second kernel: under
+//   kShortPlan us the estimate must win kAddedPass us beside the margin;
+// - a smaller tile with fewer splits reads the panels more often, in narrower
+//   rows, for the partials it saves: the rules' partials must come to kSavedShare
+//   of the panels' added bytes, and fp8 blocks, whose rows are half as long, to
+//   at most kNarrowStages stages.
+// Of 1300 shapes on MI355X (M 1..8192, N and K 64..16384, all four types) whose
+// plan the model changes, with operands from HBM, 9 ran more than 2% slower than
+// on the rules' plan (10% at most) and all 1.48x faster in geometric mean; with
+// the margin alone 67 did (45% at most: e5m2 276 x 5120 x 14592 45 us on 128 x
+// 256 tiles at 4 splits, 82 on 64 x 128 unsplit), at the same mean.
+constexpr double kAddedPass = 1.2, kShortPlan = 8.0, kSavedShare = 0.24;
+constexpr int64_t kNarrowStages = 48;
 
 }  // namespace
 
@@ -224,7 +237,7 @@ int gemm_tiled_plan(int dtype, int64_t M, int64_t N, int64_t K, const DeviceProp
     // on 128 x 128 tiles at 4 splits, 28.0 on 64 x 128 at 2).
     const int64_t rules_blocks = tiles(cfg) * splits;
     // (An unsplit pick stays with a workspace off 16 bytes, which it leaves alone.)
-    if (pinned < 0 && force_splits < 1 && !fill_rule && (splits == 1 ? scratch.on_16 : rules_blocks != cus)) {
+    if (pinned < 0 && force_splits < 1 && !fill_rule && cfg > 0 && (splits == 1 ? scratch.on_16 : rules_blocks != cus)) {
         const double a_bytes = (double)(M * K * e), b_bytes = (double)(K * N * e), outputs = (double)(M * N);
         auto estimate = [&](int c, int64_t tiles_m, int64_t tiles_n, int64_t sp, double limit) {
             const TiledLoad load{a_bytes + b_bytes + 2.0 * outputs, (double)tiles_m * b_bytes + (double)tiles_n * a_bytes,
@@ -235,12 +248,17 @@ int gemm_tiled_plan(int dtype, int64_t M, int64_t N, int64_t K, const DeviceProp
         auto partials = [&](int64_t sp) { return sp > 1 ? (size_t)(sp * M * N) * sizeof(float) : 0; };
         int best_cfg = cfg;
         int64_t best_splits = splits;
-        double best = kMargin * estimate(cfg, (M + kConfigs[cfg].bm - 1) / kConfigs[cfg].bm,
-                                         (N + kConfigs[cfg].bn - 1) / kConfigs[cfg].bn, splits, 1e30);
+        const int64_t rules_tm = (M + kConfigs[cfg].bm - 1) / kConfigs[cfg].bm;
+        const int64_t rules_tn = (N + kConfigs[cfg].bn - 1) / kConfigs[cfg].bn;
+        const double rules_us = estimate(cfg, rules_tm, rules_tn, splits, 1e30);
+        const double added_pass = splits == 1 && rules_us < kShortPlan ? kAddedPass : 0.0;
+        double best = kMargin * rules_us;
         for (int c = n128_only ? 2 : 0; c < 5; ++c) {
             // fp8 rows of 64 bytes stream a wide B poorly: e5m2 7 x 13568 x 2560
-            // 11.8 us unsplit on 64 x 64 tiles, 9.7 on 64 x 128 at 2 splits.
-            if (c == 4 && e == 1 && N > 8192) continue;
+            // 11.8 us unsplit on 64 x 64 tiles, 9.7 on 64 x 128 at 2 splits; so do
+            // rows of 128 where the rules take 256: e5m2 284 x 12272 x 4144 34.8 us
+            // on 128 x 256 tiles, 42.6 on 64 x 128.
+            if (e == 1 && N > 8192 && (c == 4 || (c == 3 && kConfigs[cfg].bn == 256))) continue;
             const int64_t tm = (M + kConfigs[c].bm - 1) / kConfigs[c].bm, tn = (N + kConfigs[c].bn - 1) / kConfigs[c].bn;
             for (int64_t sp : kSplitCounts) {
                 // More splits only add partials: past a round of blocks, or once
@@ -250,8 +268,15 @@ int gemm_tiled_plan(int dtype, int64_t M, int64_t N, int64_t K, const DeviceProp
                 // 11 x 16064 x 3968 18.5 us on 126 blocks, 14.8 on 252.
                 const int64_t blocks = tm * tn * sp;
                 if (10 * blocks < 7 * cus && blocks < rules_blocks) continue;
-                const double t = estimate(c, tm, tn, sp, best);
-                if (t < best && uneven_ok(sp)) best = t, best_cfg = c, best_splits = sp;
+                if (sp < splits && kConfigs[c].bm * kConfigs[c].bn < kConfigs[cfg].bm * kConfigs[cfg].bn) {
+                    const double added_feed = (double)(tm - rules_tm) * b_bytes + (double)(tn - rules_tn) * a_bytes;
+                    if ((double)splits * outputs * 4.0 < kSavedShare * added_feed ||
+                        (e == 1 && stages > kNarrowStages * sp))
+                        continue;
+                }
+                const double added = sp > 1 ? added_pass : 0.0;
+                const double t = estimate(c, tm, tn, sp, best - added);
+                if (t < best - added && uneven_ok(sp)) best = t + added, best_cfg = c, best_splits = sp;
             }
         }
         // A call whose workspace would not hold the new plan's partials keeps

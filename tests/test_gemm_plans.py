@@ -126,3 +126,17 @@ def test_few_row_kernel_starts_at_a_step_of_k(plans, dtype, shape, few_rows):
     # The few-row kernel's tiles are 128 K values deep, the bounds-checked kernel's one stage of 64 bytes.
     plan, = plans([(dtype, *shape, EVERYTHING)])
     assert (plan.tile_k == 128) is few_rows, plan
+
+
+@pytest.mark.parametrize("dtype, shape, tile, splits", [
+    # Measured slower on another tile or split count: longer K per block on narrower rows, a second kernel in a
+    # product of a few us, fp8 rows of 128 bytes of a wide B, 128 x 256 tiles for whole 256 x 256 panels.
+    ("float8_e5m2", (276, 5120, 14592), (128, 256), 4), ("float8_e4m3fn", (6386, 208, 10608), (128, 256), 4),
+    ("bfloat16", (304, 4608, 6144), (128, 256), 4), ("bfloat16", (26, 80, 1312), (64, 64), 1),
+    ("float8_e5m2", (284, 12272, 4144), (128, 256), 1), ("float16", (2560, 9984, 64), (256, 256), 1),
+    # Measured faster off the powers of two and off whole panels.
+    ("float8_e5m2", (16, 8192, 8384), (64, 128), 3), ("float16", (182, 3536, 1984), (64, 64), 1),
+    ("bfloat16", (25, 208, 3552), (64, 64), 28), ("bfloat16", (5984, 2048, 4864), (256, 256), 1)])
+def test_plans_by_measured_times(plans, dtype, shape, tile, splits):
+    plan, = plans([(dtype, *shape, EVERYTHING)])
+    assert ((plan.tile_m, plan.tile_n), plan.split_k) == (tile, splits), plan
