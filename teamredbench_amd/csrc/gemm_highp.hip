@@ -7,8 +7,9 @@
 // (gemm_f32_dma_kernel, gemm_f64_dma_kernel below: 95% and 93% of peak at
 // 8192^3) runs every shape within 32-bit buffer offsets, on tiles from 256 x
 // 256 (fp32) to 32 x 128, with K split over idle CUs when the caller gives a
-// workspace (highp_choose). The rest run the register-staged kernel that
-// follows, which indexes with 64 bits and stays near 80% of peak:
+// workspace (highp_choose). The rest, and a K under 16 whose rows are off 16
+// bytes, run the register-staged kernel that follows, which indexes with 64 bits
+// and stays near 80% of peak:
 //
 // Register-staged kernel. Operands come through registers into a
 // double-buffered LDS tile (one barrier per stage), and the next stage's
@@ -743,13 +744,23 @@ HighpChoice highp_choose(bool f64, int64_t M, int64_t N, int64_t K, int cus, siz
         ch.config = 1;
         return ch;
     }
+    // Rows off 16 bytes and under 16 of K: the 4-byte pieces of 128 x 128 tiles
+    // start 24 loads a wave, three stages of them, before the first MFMA, and
+    // the register-staged kernel is done earlier (fp64 280 x 4073 x 2 6.5 us
+    // against 8.9, fp32 2941 x 2939 x 5 13.5 against 17.8; of 240 such products 32
+    // ran more than 3% slower on the ring, none here; its grid holds 65535 rows of
+    // tiles). From 16 on one of 80 did, and the ring is 1.55x faster.
+    auto short_k = [&](HighpChoice c) {
+        if (c.config == 2 && c.splits == 1 && c.pieces4 && K < 16 && M <= 65535 * (int64_t)kHpBM) c.config = 0;
+        return c;
+    };
     // 128 x 128 tiles where they fill whole rounds exactly, and for K of a few
     // stages, where the tile hardly matters. fp64 with one block per CU takes
     // 128-byte rows of A (2048^3 249 against 254 us; with more blocks their
     // 128 KiB of ring leave one block per CU and run 8-9% slower).
     if ((M % 128 == 0 && N % 128 == 0 && tiles(2) % cus == 0) || (K < 128 && M >= 512)) {
         ch.config = f64 && tiles(2) <= cus && K >= 128 && fits(3, 1) ? 3 : 2;
-        return ch;
+        return short_k(ch);
     }
     // The rest: the tile and the K split that a cost model rates fastest,
     //   MFMA     = rounds x 2 * BM * BN * K / splits at the tile's share of a
@@ -797,7 +808,7 @@ HighpChoice highp_choose(bool f64, int64_t M, int64_t N, int64_t K, int cus, siz
     // reported (26.7 us fp32 and 41.9 fp64, against 65 and 123 on 128 x 128;
     // 64 x 64 tiles take 21.8 and 39.0).
     if (ch.splits == 1 && ch.config != 2 && M >= 768 && tiles(4) <= cus && fits(6, 1)) ch.config = 6;
-    return ch;
+    return short_k(ch);
 }
 
 template <typename T, int CFG, bool PIECES4>

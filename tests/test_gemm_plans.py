@@ -140,3 +140,12 @@ def test_few_row_kernel_starts_at_a_step_of_k(plans, dtype, shape, few_rows):
 def test_plans_by_measured_times(plans, dtype, shape, tile, splits):
     plan, = plans([(dtype, *shape, EVERYTHING)])
     assert ((plan.tile_m, plan.tile_n), plan.split_k) == (tile, splits), plan
+
+
+@pytest.mark.parametrize("dtype", ["float32", "float64"])
+@pytest.mark.parametrize("shape, stages", [((2941, 2939, 5), 2), ((700, 401, 15), 2), ((700, 401, 17), 4),
+                                           ((2048, 2048, 8), 4), ((9_000_000, 3, 3), 4)])
+def test_a_short_k_off_16_bytes_runs_register_staged(plans, dtype, shape, stages):
+    # Two stages: the register-staged kernel, where rows are off 16 bytes and its grid holds them; four: the ring.
+    plan, = plans([(dtype, *shape, EVERYTHING)])
+    assert plan.k_stages == stages and (plan.tile_m, plan.tile_n) == (128, 128), plan

@@ -358,6 +358,31 @@ def test_full_precision_tiles_and_splits(lib, dtype, shape, tile, splits):
         assert (np.abs(got - ref) <= bound).all(), f"workspace {ws_bytes}: off by {np.abs(got - ref).max()}"
 
 
+# The register-staged kernel's element-wise loads: the plan's own for a K under 16 with rows off 16 bytes, forced for
+# others (odd N, odd K, both; edges of its 128 x 128 tiles and of its stages of 64 bytes).
+@pytest.mark.parametrize("dtype", ["float32", "float64"])
+@pytest.mark.parametrize("shape, forced", [((700, 401, 15), False), ((1030, 129, 9), False), ((513, 515, 1), False),
+                                           ((1, 1, 1), True), ((129, 127, 33), True), ((128, 257, 64), True),
+                                           ((255, 128, 17), True), ((300, 1001, 1003), True), ((2, 3, 2049), True)])
+def test_register_staged_kernel_off_16_bytes(lib, tune, dtype, shape, forced):
+    if forced:
+        tune(gemm_highp_staged=1)
+    m, n, k = shape
+    info = lib.gemm_info(capi.DTYPES[dtype], m, n, k)
+    assert info["k_stages"] == 2 and (info["tile_m"], info["tile_n"]) == (128, 128), info
+    ops = rp.gemm_inputs(m, n, k, dtype, seed=m + n)
+    da, db = ops["a"].cuda(), ops["b"].cuda()
+    flat = torch.full((m * n + GUARD,), float("nan"), dtype=getattr(torch, dtype), device="cuda")
+    lib.gemm(capi.DTYPES[dtype], da.data_ptr(), db.data_ptr(), flat.data_ptr(), m, n, k, 1.0, 1.0, None, 0,
+             torch.cuda.current_stream().cuda_stream)
+    torch.cuda.synchronize()
+    assert torch.isnan(flat[m * n:]).all(), "the GEMM wrote past the end of C"
+    a64, b64 = ops["a"].double().numpy(), ops["b"].double().numpy()
+    ref = a64 @ b64
+    got = flat[: m * n].view(m, n).cpu().double().numpy()
+    assert (np.abs(got - ref) <= elementwise_bound(dtype, k, np.abs(ref), np.abs(a64) @ np.abs(b64)) + 1e-300).all()
+
+
 # Shapes whose B passes 2^31 bytes, with the kernel each must run on.
 BEYOND_32_BIT = [
     ("bfloat16", 65536, GENERIC),                     # B 4 GiB
