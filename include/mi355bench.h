@@ -68,7 +68,7 @@ extern "C" {
  *
  * dst, b: n elements of `dtype`; c: n elements for TRIAD, ignored (may be NULL)
  * otherwise. Any n (0 is a no-op) and any alignment: 16-byte chunks from dst's
- * first 16-byte boundary on, the elements before and after them one by one.
+ * first 128-byte line on, the elements before and after them one by one.
  * Arithmetic: fp32 math with one round-to-nearest-even to the element type
  * (fp64 math for float64); TRIAD is one fused multiply-add, fma(s, c, b).
  * blocks_per_cu: grid = min(CUs * blocks_per_cu, work); <= 0 selects the
@@ -187,9 +187,19 @@ int mb_time_gemm_rotating(int dtype, const void* const* A,
  * kind = MB_KIND_STREAM: a = op, b = dtype, m = n elements, n = blocks_per_cu.
  * kind = MB_KIND_GEMM:   a = dtype, m, n, k = shape (b ignored).
  * Beyond the reference's keys: "overrides" (the MB_TUNE_* knobs in force,
- * by name; {} normally) and, for GEMM, "workspace_bytes", "split_k" and
- * "fallback" (why a faster kernel family could not take the shape and a
- * bounds-checked kernel runs it instead; "" when none).
+ * by name; {} normally) and, for GEMM, "workspace_bytes", "split_k",
+ * "fallback" (why the kernels for rows on 16 bytes could not take the shape as
+ * it is; "" when they do) and "kernel_family", which kernels run:
+ *   "tiled"           16-bit / fp8, LDS-DMA pipeline
+ *   "repacked_tiled"  the same on operands copied to rows on 16 bytes
+ *   "few_rows"        16-bit / fp8, up to 64 rows, B through registers
+ *   "small_m"         bf16 / fp16, up to 4 rows, no matrix instructions
+ *   "bounds_checked"  16-bit / fp8, any shape
+ *   "ring"            fp32 / fp64, LDS-DMA ring, 16-byte pieces
+ *   "ring_4_byte"     the same in 4-byte pieces (rows off 16 bytes)
+ *   "register_staged" fp32 / fp64, any shape
+ * "implementation" keeps one name for all 16-bit / fp8 shapes off 16 bytes, and
+ * one for "ring_4_byte" and "register_staged"; the family tells them apart.
  * Returns MB_ERR_INVALID_ARG if json is NULL or cap is too small.
  */
 int mb_kernel_info(int kind, int a, int b, int64_t m, int64_t n, int64_t k,

@@ -482,6 +482,7 @@ int mb_kernel_info(int kind, int a, int b, int64_t m, int64_t n, int64_t k, char
         GemmPlan plan;
         if ((rc = gemm_plan(a, m, n, k, *props, Scratch{SIZE_MAX}, &plan)) != MB_OK) return rc;
         j.str("implementation", plan.implementation);
+        j.str("kernel_family", plan.family);
         j.num("threads_per_block", plan.threads);
         j.num("grid_blocks", plan.grid);
         j.num("tile_m", plan.tile_m);

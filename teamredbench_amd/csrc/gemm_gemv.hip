@@ -235,6 +235,7 @@ int gemm_gemv_plan(int dtype, int64_t M, int64_t N, int64_t K, const DeviceProps
     const int64_t force_splits = tuning(MB_TUNE_GEMM_SPLITS);
     if (force_splits >= 1) splits = force_splits;
     plan->implementation = "gfx950_gemv_stream";
+    plan->family = "small_m";
     plan->threads = kGvThreads;
     plan->grid = (int)(groups * splits);
     plan->tile_m = (int)M;

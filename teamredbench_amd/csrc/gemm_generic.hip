@@ -238,6 +238,7 @@ void launch_generic(const void* A, const void* B, void* C, int64_t M, int64_t N,
 int gemm_generic_plan(int dtype, int64_t M, int64_t N, int64_t K, GemmPlan* plan) {
     (void)K;
     plan->implementation = "gfx950_mfma_generic";
+    plan->family = "bounds_checked";
     plan->threads = kGenThreads;
     const int64_t gx = (N + kGenTile - 1) / kGenTile, gy = (M + kGenTile - 1) / kGenTile;
     plan->grid = (int)(gx * gy);

@@ -887,7 +887,9 @@ int gemm_highp_plan(int dtype, int64_t M, int64_t N, int64_t K, const DeviceProp
     plan->tile_m = t.bm;
     plan->tile_n = t.bn;
     if (ch.config != 0) {
-        // The plain name when the rows are off 16 bytes: `fallback` then says why 16-byte pieces do not reach.
+        // The plain name when the rows are off 16 bytes (`fallback` says why): the family tells the ring on
+        // 4-byte pieces from the register-staged kernel.
+        plan->family = ch.pieces4 ? "ring_4_byte" : "ring";
         plan->implementation = f64 ? (ch.pieces4 ? "gfx950_mfma_f64_16x16x4" : "gfx950_mfma_f64_16x16x4_lds_dma")
                                    : (ch.pieces4 ? "gfx950_mfma_f32_32x32x2" : "gfx950_mfma_f32_32x32x2_lds_dma");
         plan->threads = 64 * t.wgm * t.wgn;
@@ -909,6 +911,7 @@ int gemm_highp_plan(int dtype, int64_t M, int64_t N, int64_t K, const DeviceProp
         return MB_ERR_SHAPE;
     }
     plan->implementation = f64 ? "gfx950_mfma_f64_16x16x4" : "gfx950_mfma_f32_32x32x2";
+    plan->family = "register_staged";
     plan->threads = kHpThreads;
     plan->grid = (int)(gx * gy);
     plan->wave_grid_m = 2;

@@ -118,7 +118,8 @@ int gemm_packed_plan(int dtype, int64_t M, int64_t N, int64_t K, const DevicePro
     if (at > scratch) return MB_ERR_SHAPE;
     p.packed = true;
     p.workspace = at;
-    p.implementation = "gfx950_mfma_generic";
+    p.implementation = "gfx950_mfma_generic";   // the name of all shapes off 16 bytes; the family tells them apart
+    p.family = "repacked_tiled";
     p.variant = kVariantPacked;
     *plan = p;
     return MB_OK;

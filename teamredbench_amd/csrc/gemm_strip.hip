@@ -291,7 +291,8 @@ int gemm_strip_plan(int dtype, int64_t M, int64_t N, int64_t K, const DeviceProp
     const int64_t per = (steps + splits - 1) / splits;
     splits = (steps + per - 1) / per;                           // no split without a step
     *plan = GemmPlan{};
-    plan->implementation = "gfx950_mfma_generic";
+    plan->implementation = "gfx950_mfma_generic";   // as gemm_pack.hip
+    plan->family = "few_rows";
     plan->threads = 64 * kStripWaves;
     plan->grid = (int)(groups * splits);
     plan->tile_m = 16 * fm;

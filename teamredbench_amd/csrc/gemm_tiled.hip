@@ -307,6 +307,7 @@ int gemm_tiled_plan(int dtype, int64_t M, int64_t N, int64_t K, const DeviceProp
                       (mfma_force == 16 || (mfma_force != 32 && c.bm >= 128));
     const int frag = mi16 ? 16 : 32;
     plan->implementation = mi16 ? "gfx950_mfma16_lds_dma" : "gfx950_mfma32_lds_dma";
+    plan->family = "tiled";
     plan->threads = 64 * c.wgm * c.wgn;
     plan->grid = (int)(tiles(cfg) * splits);
     plan->tile_m = c.bm;

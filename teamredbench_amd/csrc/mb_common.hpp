@@ -110,6 +110,7 @@ int stream_launch(int op, int dtype, void* dst, const void* b, const void* c, ui
 
 struct GemmPlan {
     const char* implementation = "";
+    const char* family = "";    // which kernels run ("kernel_family" of mb_kernel_info)
     int threads = 0;
     int grid = 0;
     int tile_m = 0, tile_n = 0, tile_k = 0;

@@ -16,8 +16,8 @@ int main() {
     while (std::scanf("%d %" SCNd64 " %" SCNd64 " %" SCNd64 " %" SCNu64 " %d", &dtype, &m, &n, &k, &scratch, &on_16) == 6) {
         mb::GemmPlan p;
         const int rc = mb::gemm_plan(dtype, m, n, k, props, mb::Scratch{(size_t)scratch, on_16 != 0}, &p);
-        std::printf("%d %d %d %d %d %d %zu %s\n", rc, p.tile_m, p.tile_n, p.tile_k, p.k_stages, p.split_k, p.workspace,
-                    p.implementation);
+        std::printf("%d %d %d %d %d %d %zu %s %s\n", rc, p.tile_m, p.tile_n, p.tile_k, p.k_stages, p.split_k, p.workspace,
+                    p.implementation, p.family);
     }
     return 0;
 }

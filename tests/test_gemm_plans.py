@@ -24,6 +24,7 @@ class Plan(NamedTuple):
     split_k: int
     workspace: int
     implementation: str
+    family: str
 
 
 @pytest.fixture(scope="session")
@@ -41,7 +42,7 @@ def plans(tmp_path_factory):
         assert len(out) == len(shapes)
         rows = [line.split() for line in out]
         assert all(row[0] == "0" for row in rows)
-        return [Plan(*map(int, row[1:7]), row[7]) for row in rows]
+        return [Plan(*map(int, row[1:7]), *row[7:]) for row in rows]
 
     return ask
 
@@ -63,13 +64,13 @@ def _near_the_limit(dtype: str, count: int) -> list[tuple]:
 def test_full_precision_offsets_stay_in_31_bits(plans, dtype):
     # The ring's kernels form (last stage's first K) x (bytes per row of B) in 32-bit signed integers, and their
     # splits run whole stages of tile_k: every byte offset up to the last stage's end must stay below 2^31.
-    # The register-staged kernel (two stages) indexes with 64 bits.
+    # The register-staged kernel indexes with 64 bits.
     size = {"float32": 4, "float64": 8}[dtype]
     shapes = [shape for shape in _near_the_limit(dtype, 2000) if shape[0] == dtype]
     ring = 0
     for (_, m, n, k, scratch), plan in zip(shapes, plans(shapes)):
         assert plan.workspace <= scratch
-        if plan.k_stages == 2:
+        if plan.family == "register_staged":
             continue
         ring += 1
         per = -(-(-(-k // plan.tile_k)) // plan.split_k)     # stages per split
@@ -114,18 +115,17 @@ def test_the_reported_workspace_size_is_enough_at_any_address(plans):
                                              ((300, 129, 255), False), ((300, 129, 257), True), ((300, 127, 319), False),
                                              ((300, 127, 321), True), ((8192, 50257, 4096), True)])
 def test_operands_are_repacked_where_it_pays(plans, dtype, shape, repacked):
-    # The bounds-checked kernel has two stages; the pipelined ones on repacked operands have more.
     plan, = plans([(dtype, *shape, EVERYTHING)])
-    assert (plan.k_stages > 2 and plan.workspace > 0) is repacked, plan
+    assert plan.family == ("repacked_tiled" if repacked else "bounds_checked"), plan
+    assert (plan.workspace > 0) is repacked, plan
 
 
 @pytest.mark.parametrize("dtype, shape, few_rows", [
     ("bfloat16", (33, 129, 31), False), ("float16", (64, 1031, 5), False), ("bfloat16", (32, 129, 31), True),
     ("float16", (33, 129, 33), True), ("float8_e4m3fn", (64, 129, 31), True), ("bfloat16", (64, 8, 33), True)])
 def test_few_row_kernel_starts_at_a_step_of_k(plans, dtype, shape, few_rows):
-    # The few-row kernel's tiles are 128 K values deep, the bounds-checked kernel's one stage of 64 bytes.
     plan, = plans([(dtype, *shape, EVERYTHING)])
-    assert (plan.tile_k == 128) is few_rows, plan
+    assert plan.family == ("few_rows" if few_rows else "bounds_checked"), plan
 
 
 @pytest.mark.parametrize("dtype, shape, tile, splits", [
@@ -143,9 +143,9 @@ def test_plans_by_measured_times(plans, dtype, shape, tile, splits):
 
 
 @pytest.mark.parametrize("dtype", ["float32", "float64"])
-@pytest.mark.parametrize("shape, stages", [((2941, 2939, 5), 2), ((700, 401, 15), 2), ((700, 401, 17), 4),
-                                           ((2048, 2048, 8), 4), ((9_000_000, 3, 3), 4)])
-def test_a_short_k_off_16_bytes_runs_register_staged(plans, dtype, shape, stages):
-    # Two stages: the register-staged kernel, where rows are off 16 bytes and its grid holds them; four: the ring.
+@pytest.mark.parametrize("shape, family", [
+    ((2941, 2939, 5), "register_staged"), ((700, 401, 15), "register_staged"), ((700, 401, 17), "ring_4_byte"),
+    ((2048, 2048, 8), "ring"), ((9_000_000, 3, 3), "ring_4_byte")])   # (its grid does not hold those rows)
+def test_a_short_k_off_16_bytes_runs_register_staged(plans, dtype, shape, family):
     plan, = plans([(dtype, *shape, EVERYTHING)])
-    assert plan.k_stages == stages and (plan.tile_m, plan.tile_n) == (128, 128), plan
+    assert plan.family == family and (plan.tile_m, plan.tile_n) == (128, 128), plan

@@ -350,8 +350,8 @@ def test_e5m2_selects_the_e5m2_operand_format(lib):
 @pytest.mark.parametrize("shape", [(1, 1, 1), (7, 13, 5), (64, 64, 64), (129, 257, 33), (300, 200, 17),
                                    (256, 512, 1024), (130, 130, 130)])
 def test_highp_against_float64_brute_force(lib, dtype, shape):
-    # Odd K or N take the element-wise load path, multiples of 4 (fp32) / 2 (fp64) the vector path;
-    # every element must sit within the accumulation-error bound of an fp64 brute-force product.
+    # Odd K or N take the ring's 4-byte pieces (the register-staged kernel's element loads: test_gpu_gemm_ragged.py),
+    # multiples of 4 (fp32) / 2 (fp64) its 16-byte pieces; every element must sit within the accumulation-error bound of an fp64 brute-force product.
     m, n, k = shape
     print(f"[gemm] highp {dtype} {shape}", flush=True)
     ops = rp.gemm_inputs(m, n, k, dtype, seed=11)
@@ -367,13 +367,14 @@ def test_highp_against_float64_brute_force(lib, dtype, shape):
 @pytest.mark.parametrize("dtype", HIGHP)
 def test_highp_kernel_info(lib, dtype):
     # 1000^3 takes the LDS-DMA ring with partial last tiles and a ragged K; 1001 columns (rows off
-    # 16 bytes) the register-staged kernel
+    # 16 bytes) the ring in 4-byte pieces, under the register-staged kernel's name
     info = lib.gemm_info(capi.DTYPES[dtype], 1000, 1000, 1000)
     assert info["implementation"] == {"float32": "gfx950_mfma_f32_32x32x2_lds_dma",
                                       "float64": "gfx950_mfma_f64_16x16x4_lds_dma"}[dtype]
-    assert info["workspace_bytes"] == 0 and info["tile_m"] == 128
+    assert info["workspace_bytes"] == 0 and info["tile_m"] == 128 and info["kernel_family"] == "ring"
     info = lib.gemm_info(capi.DTYPES[dtype], 1000, 1001, 1000)
     assert info["implementation"] == {"float32": "gfx950_mfma_f32_32x32x2", "float64": "gfx950_mfma_f64_16x16x4"}[dtype]
+    assert info["kernel_family"] == "ring_4_byte"
 
 
 @pytest.mark.parametrize("shape, tile", [((4096, 4096, 64), (256, 256)), ((8192, 2048, 96), (256, 256)),
@@ -388,10 +389,11 @@ def test_f32_lds_dma_kernel_selection(lib, shape, tile):
     # no more than the 128 x 128 tiles' at 0.975 of the rate (4352 x 4096: 2 rounds of 272 large tiles
     # against 5 of 1088 small; 6144^2: 3 against 9), else 128 x 128 tiles (2048^3: 64 large tiles, 256
     # small), partial last tiles included; a K off the 16-deep stage runs whole stages. Rows of A or B
-    # off 16 bytes keep the register-staged kernel.
+    # off 16 bytes take 128 x 128 tiles in 4-byte pieces.
     info = lib.gemm_info(capi.DT_FLOAT32, *shape)
     if tile is None:
         assert info["implementation"] == "gfx950_mfma_f32_32x32x2" and info["tile_m"] == 128
+        assert info["kernel_family"] == "ring_4_byte"
     else:
         assert info["implementation"] == "gfx950_mfma_f32_32x32x2_lds_dma"
         assert (info["tile_m"], info["tile_n"]) == tile
@@ -415,7 +417,8 @@ def test_f32_lds_dma_against_float64_brute_force(lib, shape, tune):
     bound = ref.abs() * UNIT["float32"] + (k + 1) * UNIT["float32"] * mag
     assert torch.all((got - ref).abs() <= bound)
     tune(gemm_highp_staged=1)
-    assert lib.gemm_info(capi.DT_FLOAT32, m, n, k)["implementation"] == "gfx950_mfma_f32_32x32x2"
+    info = lib.gemm_info(capi.DT_FLOAT32, m, n, k)
+    assert info["implementation"] == "gfx950_mfma_f32_32x32x2" and info["kernel_family"] == "register_staged"
     staged = _gemm(lib, "float32", ops["a"], ops["b"]).double()
     assert torch.all((staged - ref).abs() <= bound)
 
@@ -427,10 +430,11 @@ def test_f32_lds_dma_against_float64_brute_force(lib, shape, tune):
                                          ((4096, 8001, 64), None), ((4096, 8192, 61), None)])
 def test_f64_lds_dma_kernel_selection(lib, shape, tile):
     # fp64: 128 x 128 tiles for every shape the ring takes (two blocks per CU), partial last tiles and a
-    # K off the 8-deep stage included; rows of A or B off 16 bytes keep the register-staged kernel.
+    # K off the 8-deep stage included; rows of A or B off 16 bytes take the same tiles in 4-byte pieces.
     info = lib.gemm_info(capi.DT_FLOAT64, *shape)
     if tile is None:
         assert info["implementation"] == "gfx950_mfma_f64_16x16x4" and info["tile_m"] == 128
+        assert info["kernel_family"] == "ring_4_byte"
     else:
         assert info["implementation"] == "gfx950_mfma_f64_16x16x4_lds_dma"
         assert (info["tile_m"], info["tile_n"]) == tile
@@ -452,7 +456,8 @@ def test_f64_lds_dma_against_float64_brute_force(lib, shape, tune):
     bound = ref.abs() * UNIT["float64"] + (k + 1) * UNIT["float64"] * mag
     assert torch.all((got - ref).abs() <= bound)
     tune(gemm_highp_staged=1)
-    assert lib.gemm_info(capi.DT_FLOAT64, m, n, k)["implementation"] == "gfx950_mfma_f64_16x16x4"
+    info = lib.gemm_info(capi.DT_FLOAT64, m, n, k)
+    assert info["implementation"] == "gfx950_mfma_f64_16x16x4" and info["kernel_family"] == "register_staged"
     staged = _gemm(lib, "float64", ops["a"], ops["b"])
     assert torch.all((staged - ref).abs() <= bound)
 
@@ -689,7 +694,7 @@ def test_overrides_are_reported_and_the_environment_is_ignored(lib, tune, monkey
     ("bfloat16", (256, 256, 256), "gfx950_mfma32_lds_dma", ""),
 ])
 def test_kernel_info_names_the_fallback(lib, dtype, shape, impl, reason):
-    # A shape the pipelined kernels cannot take runs on a bounds-checked kernel, and the plan says why.
+    # A shape whose rows keep it off the 16-byte kernels as it is runs another, and the plan says why.
     info = lib.gemm_info(capi.DTYPES[dtype], *shape)
     assert info["implementation"].startswith(impl) and info["fallback"] == reason
     _check_random(lib, dtype, *shape, seed=1)

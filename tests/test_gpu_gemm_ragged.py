@@ -1,5 +1,5 @@
 """GEMM shapes off the tile grid (-m gpu): a ragged N or K on the pipelined
-kernels, and the bounds-checked kernel that takes what they cannot.
+kernels, and the kernels that take what those cannot.
 
 N that is not a multiple of the tile width but keeps B's rows on 16 bytes (a
 multiple of 8 for 16-bit inputs, of 16 for fp8) runs the LDS-DMA kernels with
@@ -24,9 +24,11 @@ as zeros; the same checks hold, with the last split of a split-K plan running
 past K, and with N ragged too.
 
 Shapes whose A or B rows are not on 16 bytes (K or N not a multiple of 8, of
-16 for fp8) run the bounds-checked kernel
-(128 x 128 tiles, every global access checked); the same checks hold there,
-on its 16-byte and element-wise A paths, and on aligned shapes forced onto it.
+16 for fp8) run the pipelined kernels on repacked operands, the few-row kernel
+(up to 64 rows of A) or, for a short K or without a workspace, the
+bounds-checked kernel (128 x 128 tiles, every global access checked); the same
+checks hold there, on its 16-byte and element-wise A paths, and on aligned
+shapes forced onto it.
 """
 from __future__ import annotations
 
@@ -211,20 +213,21 @@ def test_workspace_off_16_bytes(lib, dtype, shape, uses_it, offset):
     assert (np.abs(got - ref) <= elementwise_bound(dtype, k, np.abs(ref), scale * (np.abs(a64) @ np.abs(b64)))).all()
 
 
-GENERIC = "gfx950_mfma_generic"
-# (dtype, (M, N, K)): B rows off 16 bytes, or A rows off 16 bytes (K not a multiple of 8 / 16).
+GENERIC = "gfx950_mfma_generic"   # one name for every kernel of rows off 16 bytes; the family says which runs
+# (dtype, (M, N, K), family): B rows off 16 bytes, or A rows off 16 bytes (K not a multiple of 8 / 16).
 FALLBACKS = [
-    ("bfloat16", (300, 1001, 520)), ("bfloat16", (257, 4000, 1001)), ("bfloat16", (128, 50257, 256)),
-    ("bfloat16", (1, 7, 3)), ("float16", (33, 129, 65)), ("float16", (520, 2050, 1001)),
-    ("float8_e4m3fn", (200, 1000, 4000)), ("float8_e4m3fn", (130, 2048, 4001)), ("float8_e5m2", (77, 4104, 1000)),
-    ("float8_e5m2", (129, 257, 97)),
+    ("bfloat16", (300, 1001, 520), "repacked_tiled"), ("bfloat16", (257, 4000, 1001), "repacked_tiled"),
+    ("bfloat16", (128, 50257, 256), "repacked_tiled"), ("bfloat16", (1, 7, 3), "bounds_checked"),
+    ("float16", (33, 129, 65), "few_rows"), ("float16", (520, 2050, 1001), "repacked_tiled"),
+    ("float8_e4m3fn", (200, 1000, 4000), "repacked_tiled"), ("float8_e4m3fn", (130, 2048, 4001), "repacked_tiled"),
+    ("float8_e5m2", (77, 4104, 1000), "repacked_tiled"), ("float8_e5m2", (129, 257, 97), "bounds_checked"),
 ]
 
 
-@pytest.mark.parametrize("dtype, shape", FALLBACKS)
-def test_shapes_off_the_pipelined_kernels(lib, dtype, shape):
+@pytest.mark.parametrize("dtype, shape, family", FALLBACKS)
+def test_shapes_off_the_pipelined_kernels(lib, dtype, shape, family):
     info = run_checked(lib, dtype, *shape, seed=sum(shape))
-    assert info["implementation"] == GENERIC and info["fallback"] != "", info
+    assert info["implementation"] == GENERIC and info["fallback"] != "" and info["kernel_family"] == family, info
 
 
 # Rows off 16 bytes: N off, K off, both, by one element either side of a multiple; one row; a K shorter than a
@@ -233,10 +236,13 @@ def test_shapes_off_the_pipelined_kernels(lib, dtype, shape):
 @pytest.mark.parametrize("shape", [(300, 513, 512), (300, 512, 511), (257, 255, 1025), (64, 1030, 4099),
                                    (1, 1025, 2049), (40, 2047, 3), (520, 130, 77), (1024, 1279, 1281)])
 def test_rows_off_16_bytes(lib, dtype, shape):
-    # The same operands with the workspace the plan asks for (repacked) and without one (bounds-checked kernel).
+    # The same operands with the workspace the plan asks for (repacked from K = 256 on) and without one
+    # (bounds-checked kernel; up to 64 rows the few-row kernel either way, 16-bit ones of 33 rows from K = 32 on).
     m, n, k = shape
     dt = capi.DTYPES[dtype]
-    run_checked(lib, dtype, *shape, seed=m)
+    info = run_checked(lib, dtype, *shape, seed=m)
+    few = m <= 64 and (m <= 32 or k >= 32 or dtype.startswith("float8"))
+    assert info["kernel_family"] == ("few_rows" if few else "repacked_tiled" if k >= 256 else "bounds_checked"), info
     ops = rp.gemm_inputs(m, n, k, dtype, seed=m)
     da, db = ops["a"].cuda(), ops["b"].cuda()
     flat = torch.full((m * n + GUARD,), float("nan"), dtype=rp.gemm_output_dtype(dtype), device="cuda")
@@ -261,7 +267,9 @@ def test_few_rows_off_16_bytes(lib, tune, dtype, splits, shape):
     m, n, k = shape
     dt = capi.DTYPES[dtype]
     tune(gemm_splits=splits)
-    run_checked(lib, dtype, *shape, seed=m + n)
+    info = run_checked(lib, dtype, *shape, seed=m + n)
+    # 9 columns are fewer than a lane of one fragment of fp8 takes (16).
+    assert info["kernel_family"] == ("bounds_checked" if n == 9 and dtype.startswith("float8") else "few_rows"), info
     ops = rp.gemm_inputs(m, n, k, dtype, seed=m + n)
     da, db = ops["a"].cuda(), ops["b"].cuda()
     a64, b64 = ops["a"].double().numpy(), ops["b"].double().numpy()
@@ -287,7 +295,7 @@ def test_few_rows_off_16_bytes(lib, tune, dtype, splits, shape):
 def test_bounds_checked_kernel_forced(lib, tune, dtype, shape):
     tune(gemm_force_generic=1)
     info = run_checked(lib, dtype, *shape, seed=len(shape) + shape[0])
-    assert info["implementation"] == GENERIC, info
+    assert info["implementation"] == GENERIC and info["kernel_family"] == "bounds_checked", info
 
 
 @pytest.mark.parametrize("dtype", ["float32", "float64"])
@@ -369,7 +377,7 @@ def test_register_staged_kernel_off_16_bytes(lib, tune, dtype, shape, forced):
         tune(gemm_highp_staged=1)
     m, n, k = shape
     info = lib.gemm_info(capi.DTYPES[dtype], m, n, k)
-    assert info["k_stages"] == 2 and (info["tile_m"], info["tile_n"]) == (128, 128), info
+    assert info["kernel_family"] == "register_staged", info
     ops = rp.gemm_inputs(m, n, k, dtype, seed=m + n)
     da, db = ops["a"].cuda(), ops["b"].cuda()
     flat = torch.full((m * n + GUARD,), float("nan"), dtype=getattr(torch, dtype), device="cuda")

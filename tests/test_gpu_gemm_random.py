@@ -3,7 +3,7 @@
 The fixed-shape tests pin each kernel and plan branch; these shapes are drawn
 at random (M 1..2000, N and K multiples of 128 / 64, of 8, or arbitrary) so that
 the plan's choices -- small-M stream kernel, tile configuration, K split count
-up to 32, bounds-checked generic kernel -- are exercised where no test chose
+up to 32, the kernels of rows off 16 bytes -- are exercised where no test chose
 them. Every element of C is checked against an fp64 matmul of the same
 operands (the fp8 codes' exact values, times scale_a * scale_b) within its
 rounding bound: the output rounding of C's type, the fp32 rounding of the fp8
@@ -35,6 +35,7 @@ pytestmark = pytest.mark.gpu
 IMPLEMENTATIONS = {"gfx950_gemv_stream", "gfx950_mfma16_lds_dma", "gfx950_mfma32_lds_dma", "gfx950_mfma_generic",
                    "gfx950_mfma_f32_32x32x2", "gfx950_mfma_f32_32x32x2_lds_dma", "gfx950_mfma_f64_16x16x4",
                    "gfx950_mfma_f64_16x16x4_lds_dma"}
+FAMILIES = {"small_m", "tiled", "repacked_tiled", "few_rows", "bounds_checked", "ring", "ring_4_byte", "register_staged"}
 DTYPES = ["bfloat16", "float16", "float8_e4m3fn", "float8_e5m2", "float32", "float64"]
 def _dim(rng: np.random.Generator, aligned: int, hi: int) -> int:
     kind = rng.random()
@@ -68,7 +69,7 @@ def test_planned_gemm_on_random_shapes(lib, dtype, case):
     info = lib.gemm_info(dt, m, n, k)
     print(f"[gemm-random] {dtype} {m}x{n}x{k} case {case}: {info['implementation']} "
           f"{info['tile_m']}x{info['tile_n']} split {info['split_k']}", flush=True)
-    assert info["implementation"] in IMPLEMENTATIONS, info
+    assert info["implementation"] in IMPLEMENTATIONS and info["kernel_family"] in FAMILIES, info
     ops = rp.gemm_inputs(m, n, k, dtype, seed=case)
     da, db = ops["a"].cuda(), ops["b"].cuda()
     dc = torch.full((m, n), float("nan"), dtype=rp.gemm_output_dtype(dtype), device="cuda")

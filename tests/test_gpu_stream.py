@@ -73,7 +73,7 @@ def test_stream_configuration_sizes(lib, mode, dtype):
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
 @pytest.mark.parametrize("mode", MODES)
 @pytest.mark.parametrize("offset", [1, 3])
-def test_unaligned_buffers_take_the_scalar_kernel(lib, mode, dtype, offset):
+def test_unaligned_buffers(lib, mode, dtype, offset):
     n = 50_001
     print(f"[stream] unaligned {mode} {dtype} offset={offset}", flush=True)
     b, c = rp.stream_inputs(n, dtype, seed=offset)
