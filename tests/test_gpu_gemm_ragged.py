@@ -257,6 +257,23 @@ def test_rows_off_16_bytes(lib, dtype, shape):
     assert (np.abs(got - ref) <= elementwise_bound(dtype, k, np.abs(ref), scale * (np.abs(a64) @ np.abs(b64)))).all()
 
 
+# Repacked operands on every tile: N and K off, columns past the last whole 8 (7, 1 and 5 of them, 9 in all), partial
+# last tiles of rows, K splits that are equal or not, and for fp8 an even stage count per split, which takes the
+# 16x16x128 kernel on tiles of 128 rows and more.
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("config, splits", [(0, 1), (1, 1), (2, 1), (3, 1), (4, 1), (1, 3), (2, 3), (3, 3), (4, 3)])
+@pytest.mark.parametrize("shape", [(300, 1031, 1029), (333, 777, 1001), (515, 261, 2301), (70, 9, 257)])
+def test_repacked_operands_on_every_tile(lib, tune, dtype, config, splits, shape):
+    tune(gemm_tiled_config=config, gemm_splits=splits)
+    info = run_checked(lib, dtype, *shape, seed=config + sum(shape))
+    tile = [(256, 256), (128, 256), (128, 128), (64, 128), (64, 64)][config]
+    assert info["kernel_family"] == "repacked_tiled" and (info["tile_m"], info["tile_n"]) == tile, info
+    stages = -(-shape[2] // (64 if dtype.startswith("float8") else 32))
+    assert info["split_k"] == splits
+    if dtype.startswith("float8") and config <= 2:
+        assert info["frag_m"] == (16 if -(-stages // splits) % 2 == 0 else 32), info
+
+
 # Few rows with N or K off 16 bytes: every count of 16-row fragments and its edges, the narrowest N a lane's
 # columns fit, one column past a block, K of one partial step, whole steps only, a partial one after them.
 @pytest.mark.parametrize("dtype", DTYPES)
