@@ -123,7 +123,7 @@ int mb_gemm(int dtype, const void* A, const void* B, void* C, int64_t M,
             int64_t N, int64_t K, float scale_a, float scale_b, void* workspace,
             size_t workspace_bytes, void* stream);
 
-/* Workspace bytes mb_gemm needs for this dtype and shape (0 if none). */
+/* Workspace bytes mb_gemm uses for this dtype and shape (0 if none). */
 size_t mb_gemm_workspace_size(int dtype, int64_t M, int64_t N, int64_t K);
 
 /*

@@ -89,7 +89,7 @@ int gemm_tiled_launch_e5m2(const GemmPlan& plan, const void* A, const void* B, v
 int gemm_generic_launch(int dtype, const void* A, const void* B, void* C, int64_t M, int64_t N,
                         int64_t K, float alpha, hipStream_t stream);
 // The tiled kernels on repacked operands, for rows off 16 bytes: MB_ERR_SHAPE
-// when they cannot take the shape, would not pay, or need more than `scratch`.
+// when they cannot take the shape, K is too short to pay for the copy, or they need more than `scratch`.
 int gemm_packed_plan(int dtype, int64_t M, int64_t N, int64_t K, const DeviceProps& props, size_t scratch,
                      GemmPlan* plan);
 int gemm_packed_launch(int dtype, const void* A, const void* B, void* C, int64_t M, int64_t N, int64_t K,

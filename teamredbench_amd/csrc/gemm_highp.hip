@@ -805,8 +805,10 @@ HighpChoice highp_choose(bool f64, int64_t M, int64_t N, int64_t K, int cus, siz
         ch.config = 3;
     // One unsplit round of at least six 128-row panels runs 128 x 32 tiles:
     // 128-row tiles without a workspace are what a plan of 1000^3 has always
-    // reported (26.7 us fp32 and 41.9 fp64, against 65 and 123 on 128 x 128;
-    // 64 x 64 tiles take 21.8 and 39.0).
+    // reported (26.7 us fp32 and 41.9 fp64, against 65 and 123 on 128 x 128). No
+    // time speaks for it: 64 x 64 tiles take 21.4 and 38.6, and over 25 such shapes
+    // the pick above is 1.27x faster in geometric mean (fp32 1.07-1.45x, fp64
+    // 0.93-1.19x, the tall ones of few columns slower on it).
     if (ch.splits == 1 && ch.config != 2 && M >= 768 && tiles(4) <= cus && fits(6, 1)) ch.config = 6;
     return short_k(ch);
 }

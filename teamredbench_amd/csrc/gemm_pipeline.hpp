@@ -74,11 +74,15 @@ __device__ __forceinline__ void lds_dma(__amdgpu_buffer_rsrc_t rsrc, unsigned ld
 // tile) pairs, split by split, a split's tiles in groups of `group_m` tile
 // rows: its concurrent tiles form a compact patch of a split, whose A and B
 // panels its L2 shares, whatever the counts. A power of two keeps the splits
-// of a tile adjacent: the XCDs then divide the splits among them already (fp16
-// 16 x 8192 x 8192 at 4 splits 28.1 us so, 29.0 in runs). On MI355X, tile
-// counts that are no multiple of 8, dealt out over the XCDs before: 1.05x in
-// geometric mean over 970 unsplit bf16 / fp16 / fp8 plans, multiples of 8
-// (the same map) 1.02x in the same runs; 5740 odd splits 1.04x.
+// of a tile adjacent: up to 8 of them, the XCDs then divide the splits among
+// them already. Over 349 plans of 2 to 32 splits on MI355X (1 to 512 tiles of
+// 64 x 64 to 128 x 256, operands from HBM) either order is within 1.2% of the
+// other in geometric mean, except with tile counts that are multiples of 8, as
+// the plan's own few-row picks are: adjacent splits 2.4% faster at 4, 1.2% at 8,
+// 3.2% at 16, equal at 2, 1.7% slower at 32. Tile counts that are no multiple of
+// 8, dealt out over the XCDs before: 1.05x in geometric mean over 970 unsplit
+// bf16 / fp16 / fp8 plans, multiples of 8 (the same map) 1.02x in the same runs;
+// 5740 odd splits 1.04x.
 __device__ __forceinline__ void block_coords(int b, int tiles_m, int tiles_n, int splits, int group_m, int* tm,
                                              int* tn, int* split) {
     const int tiles = tiles_m * tiles_n;
