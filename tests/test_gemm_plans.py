@@ -81,6 +81,27 @@ def test_full_precision_offsets_stay_in_31_bits(plans, dtype):
     assert ring > len(shapes) // 2
 
 
+@pytest.mark.parametrize("dtype, size", [("bfloat16", 2), ("float8_e5m2", 1)])
+def test_tiled_offsets_stay_in_31_bits(plans, dtype, size):
+    # The same of the pipelined kernels, whose unequal K splits run whole stages of 64 bytes past K.
+    rng = random.Random(size)
+    shapes = []
+    while len(shapes) < 2000:
+        n = 16 * int(32 * 64 ** rng.random())
+        k = (LIMIT // size // n - rng.randrange(400)) // 16 * 16
+        if k > 0 and (k + 64) * 256 * size < LIMIT:
+            shapes.append((dtype, rng.choice((1, 9, 40, 130, 700)), n, k, rng.choice((0, 1 << 22, EVERYTHING))))
+    tiled = 0
+    for (_, m, n, k, scratch), plan in zip(shapes, plans(shapes)):
+        if plan.family != "tiled":
+            continue
+        tiled += 1
+        per = -(-(-(-k // plan.tile_k)) // plan.split_k)
+        assert (per * plan.split_k * plan.tile_k * n + plan.tile_n) * size < LIMIT, (m, n, k, scratch, plan)
+        assert (plan.split_k - 1) * per * plan.tile_k < k, "a split without a stage"
+    assert tiled > len(shapes) // 3
+
+
 OFF_16_WORKSPACE = [
     ("bfloat16", 300, 513, 512), ("float8_e4m3fn", 300, 1031, 1029), ("float16", 40, 2047, 4099),   # repacked, few rows
     ("float32", 5, 4099, 2051), ("float64", 600, 704, 1904), ("float32", 1000, 1500, 2000),          # K splits
