@@ -747,11 +747,13 @@ HighpChoice highp_choose(bool f64, int64_t M, int64_t N, int64_t K, int cus, siz
     // Rows off 16 bytes and under 16 of K: the 4-byte pieces of 128 x 128 tiles
     // start 24 loads a wave, three stages of them, before the first MFMA, and
     // the register-staged kernel is done earlier (fp64 280 x 4073 x 2 6.5 us
-    // against 8.9, fp32 2941 x 2939 x 5 13.5 against 17.8; of 240 such products 32
-    // ran more than 3% slower on the ring, none here; its grid holds 65535 rows of
-    // tiles). From 16 on one of 80 did, and the ring is 1.55x faster.
+    // against 8.9, fp32 2941 x 2939 x 5 13.5 against 17.8; of 779 products off 16
+    // bytes 93 ran more than 3% slower than there before this rule, none with it; its
+    // grid holds 65535 rows of tiles). From 16 to 31 one of 121 does, and the ring
+    // is 1.49x faster.
     auto short_k = [&](HighpChoice c) {
-        if (c.config == 2 && c.splits == 1 && c.pieces4 && K < 16 && M <= 65535 * (int64_t)kHpBM) c.config = 0;
+        if ((c.config == 2 || c.config == 3) && c.splits == 1 && c.pieces4 && K < 16 && M <= 65535 * (int64_t)kHpBM)
+            c.config = 0;
         return c;
     };
     // 128 x 128 tiles where they fill whole rounds exactly, and for K of a few

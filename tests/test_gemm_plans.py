@@ -170,3 +170,9 @@ def test_plans_by_measured_times(plans, dtype, shape, tile, splits):
 def test_a_short_k_off_16_bytes_runs_register_staged(plans, dtype, shape, family):
     plan, = plans([(dtype, *shape, EVERYTHING)])
     assert plan.family == family and (plan.tile_m, plan.tile_n) == (128, 128), plan
+
+
+def test_a_short_k_off_16_bytes_with_few_rows_runs_register_staged(plans):
+    # fp64 of a few 128 x 128 tiles, which the cost model picks and gives 128-byte rows of A.
+    shapes = [(280, 4073, 2), (465, 2511, 3), (462, 2769, 7), (400, 4001, 13)]
+    assert [p.family for p in plans([("float64", *s, EVERYTHING) for s in shapes])] == ["register_staged"] * 4
