@@ -7,8 +7,8 @@
 // (gemm_f32_dma_kernel, gemm_f64_dma_kernel below: 95% and 93% of peak at
 // 8192^3) runs every shape within 32-bit buffer offsets, on tiles from 256 x
 // 256 (fp32) to 32 x 128, with K split over idle CUs when the caller gives a
-// workspace (highp_choose). The rest, and a K under 16 whose rows are off 16
-// bytes, run the register-staged kernel that follows, which indexes with 64 bits
+// workspace (highp_choose). The rest, and some products of a short K (under 16,
+// 24), run the register-staged kernel that follows, which indexes with 64 bits
 // and stays near 80% of peak:
 //
 // Register-staged kernel. Operands come through registers into a
@@ -744,23 +744,31 @@ HighpChoice highp_choose(bool f64, int64_t M, int64_t N, int64_t K, int cus, siz
         ch.config = 1;
         return ch;
     }
-    // Rows off 16 bytes and under 16 of K: the 4-byte pieces of 128 x 128 tiles
-    // start 24 loads a wave, three stages of them, before the first MFMA, and
-    // the register-staged kernel is done earlier (fp64 280 x 4073 x 2 6.5 us
-    // against 8.9, fp32 2941 x 2939 x 5 13.5 against 17.8; of 779 products off 16
-    // bytes 93 ran more than 3% slower than there before this rule, none with it; its
-    // grid holds 65535 rows of tiles). From 16 to 31 one of 121 does, and the ring
-    // is 1.49x faster.
+    // Under 16 of K the register-staged kernel is done before the ring's three
+    // stages of loads are: with rows off 16 bytes on 128 x 128 tiles, whose 4-byte
+    // pieces are 24 loads a wave (fp64 280 x 4073 x 2 6.5 us against 8.9; of 779
+    // products off 16 bytes 93 ran more than 3% slower than there before this rule,
+    // none with it; from 16 on the ring is 1.5x faster), and in fp32 with more than
+    // a round of them (1570 x 2668 x 4 8.2 us against 10.3, 2941 x 2939 x 5 13.5
+    // against 17.8; 18 such products on 16 bytes 1.20x faster; off 16 bytes up to
+    // 24 of K, 4000 x 3630 x 16 18.0 against 21.7). Its grid holds 65535 rows of
+    // tiles.
     auto short_k = [&](HighpChoice c) {
-        if ((c.config == 2 || c.config == 3) && c.splits == 1 && c.pieces4 && K < 16 && M <= 65535 * (int64_t)kHpBM)
+        const bool crowded = !f64 && tiles(2) > cus;
+        if (c.config == 2 && c.splits == 1 && M <= 65535 * (int64_t)kHpBM && K < (c.pieces4 && crowded ? 24 : 16) &&
+            (c.pieces4 || crowded)) {
             c.config = 0;
+            if (!c.pieces4) *why = "K is under 16";
+        }
         return c;
     };
     // 128 x 128 tiles where they fill whole rounds exactly, and for K of a few
-    // stages, where the tile hardly matters. fp64 with one block per CU takes
+    // stages, where the tile hardly matters (under one, up to 64 of them leave
+    // the CUs idle: 64 x 64 tiles 1.1-1.6x faster). fp64 with one block per CU takes
     // 128-byte rows of A (2048^3 249 against 254 us; with more blocks their
     // 128 KiB of ring leave one block per CU and run 8-9% slower).
-    if ((M % 128 == 0 && N % 128 == 0 && tiles(2) % cus == 0) || (K < 128 && M >= 512)) {
+    const bool few_stages = K < 128 && M >= 512 && (K >= 16 || ch.pieces4 || tiles(2) > 64);
+    if ((M % 128 == 0 && N % 128 == 0 && tiles(2) % cus == 0) || few_stages) {
         ch.config = f64 && tiles(2) <= cus && K >= 128 && fits(3, 1) ? 3 : 2;
         return short_k(ch);
     }
@@ -801,8 +809,8 @@ HighpChoice highp_choose(bool f64, int64_t M, int64_t N, int64_t K, int cus, siz
             if (best < 0.0 || t < best) best = t, ch.config = c, ch.splits = sp;
         }
     }
-    // fp64 alone on a CU: 128-byte rows of A (above).
-    if (f64 && ch.config == 2 && tiles(2) * ch.splits <= cus && k_len(3, ch.splits) * (ch.splits - 1) < K &&
+    // fp64 alone on a CU: 128-byte rows of A (above), unless K leaves a row empty (378 x 4062 x 2 6.4 us, 7.9 so).
+    if (f64 && ch.config == 2 && K >= 16 && tiles(2) * ch.splits <= cus && k_len(3, ch.splits) * (ch.splits - 1) < K &&
         fits(3, ch.splits))
         ch.config = 3;
     // One unsplit round of at least six 128-row panels runs 128 x 32 tiles:
@@ -811,7 +819,7 @@ HighpChoice highp_choose(bool f64, int64_t M, int64_t N, int64_t K, int cus, siz
     // time speaks for it: 64 x 64 tiles take 21.4 and 38.6, and over 25 such shapes
     // the pick above is 1.27x faster in geometric mean (fp32 1.07-1.45x, fp64
     // 0.93-1.19x, the tall ones of few columns slower on it).
-    if (ch.splits == 1 && ch.config != 2 && M >= 768 && tiles(4) <= cus && fits(6, 1)) ch.config = 6;
+    if (ch.splits == 1 && ch.config != 2 && M >= 768 && K >= 16 && tiles(4) <= cus && fits(6, 1)) ch.config = 6;
     return short_k(ch);
 }
 

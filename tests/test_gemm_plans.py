@@ -166,6 +166,7 @@ def test_plans_by_measured_times(plans, dtype, shape, tile, splits):
 @pytest.mark.parametrize("dtype", ["float32", "float64"])
 @pytest.mark.parametrize("shape, family", [
     ((2941, 2939, 5), "register_staged"), ((700, 401, 15), "register_staged"), ((700, 401, 17), "ring_4_byte"),
+    ((4000, 3630, 25), "ring_4_byte"),
     ((2048, 2048, 8), "ring"), ((9_000_000, 3, 3), "ring_4_byte")])   # (its grid does not hold those rows)
 def test_a_short_k_off_16_bytes_runs_register_staged(plans, dtype, shape, family):
     plan, = plans([(dtype, *shape, EVERYTHING)])
@@ -176,3 +177,18 @@ def test_a_short_k_off_16_bytes_with_few_rows_runs_register_staged(plans):
     # fp64 of a few 128 x 128 tiles, which the cost model picks and gives 128-byte rows of A.
     shapes = [(280, 4073, 2), (465, 2511, 3), (462, 2769, 7), (400, 4001, 13)]
     assert [p.family for p in plans([("float64", *s, EVERYTHING) for s in shapes])] == ["register_staged"] * 4
+
+
+@pytest.mark.parametrize("dtype, shape, family, tile", [
+    # Rows on 16 bytes and under one stage of K: more than a round of 128 x 128 fp32 tiles, a round and less, few.
+    ("float32", (1570, 2668, 4), "register_staged", (128, 128)), ("float32", (2048, 2048, 12), "ring", (128, 128)),
+    ("float32", (1882, 152, 4), "ring", (64, 64)), ("float32", (1570, 2668, 16), "ring", (128, 128)),
+    ("float64", (1570, 2668, 4), "ring", (128, 128)), ("float64", (1111, 2026, 8), "ring", (128, 128)),
+    ("float64", (700, 400, 2), "ring", (64, 64))])
+def test_a_short_k_on_16_bytes(plans, dtype, shape, family, tile):
+    plan, = plans([(dtype, *shape, EVERYTHING)])
+    assert plan.family == family and (plan.tile_m, plan.tile_n) == tile, plan
+    more, = plans([("float32", 4000, 3630, 23, EVERYTHING)])   # off 16 bytes the line lies at 24 for such tiles
+    assert more.family == "register_staged", more
+    few, = plans([("float64", 378, 4062, 2, EVERYTHING)])   # 64-byte rows of A: no stage of 16 for 2 of K
+    assert few.tile_k == 8, few
